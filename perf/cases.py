@@ -99,7 +99,7 @@ def draw(rng):
         heads = rng.choice([SMALL, WIDE7])
         hi = logint(1024, 4096)
         return _case(work, heads, q=rng.choice(["bf16", "fp16"]),
-                     batch=rng.randint(3, 32 if heads == SMALL else 16), hi=hi,
+                     batch=rng.randint(3, 32 if heads == SMALL else 16), lo=hi // 4, hi=hi,
                      layers=rng.randint(8, 24), lens=lens)
     if work == "decode":
         hi = logint(2048, 16384)
