@@ -57,6 +57,7 @@ typedef enum msattn_route {
   MSATTN_ROUTE_STREAMK = 4,          /* MFMA stream-K decode kernel, then the merge kernel */
   MSATTN_ROUTE_GENERIC = 5,          /* generic VALU kernel, then the merge kernel */
   MSATTN_ROUTE_PREFILL_STREAMK = 6,  /* prefill kernel, stream-K schedule (merge in-kernel) */
+  MSATTN_ROUTE_PREFILL_ANY = 7,      /* any-layout prefill kernel (and its fold launch, if any) */
 } msattn_route;
 
 /* ABI version (MSATTN_ABI_VERSION). No reference counterpart. */

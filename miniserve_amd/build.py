@@ -49,6 +49,9 @@ FILE_FLAGS = {
     "prefill_mfma_fp8.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
     "prefill_mfma_f32kv.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
 }
+# The any-layout prefill kernels do the same.
+FILE_FLAGS.update({f"prefill_any_{q}_{kv}.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]
+                   for q in ("f32", "f16", "bf16") for kv in ("f32", "f16", "bf16", "fp8")})
 
 
 def _run(cmd: list[str]) -> None:

@@ -9,6 +9,7 @@
 
 #include "decode_mfma.h"
 #include "decode_streamk.h"
+#include "prefill_any.h"
 #include "prefill_mfma.h"
 #include "kernels.h"
 #include "msattn.h"
@@ -189,6 +190,15 @@ constexpr int kSkMinChunk = MSATTN_SK_MIN_CHUNK;  // stream-K: smallest chunk (t
 
 int mfma_rows_per_tile(int rows_per_kvh) { return rows_per_kvh >= 16 ? 16 : next_pow2(rows_per_kvh); }
 
+// A multi-token query of more than 16 rows per KV head that the copying prefill kernel cannot
+// take may run on the any-layout prefill kernel (prefill_any.h): its geometry.
+constexpr int64_t kPaReserve = 40 << 20;  // bytes of share partials a workspace reserves
+
+bool prefill_any_ok(int batch, int q_len, int num_heads, int num_kv_heads, int head_dim) {
+  return q_len > 1 && head_dim <= kMaxHeadDim && batch <= 65535 &&
+         static_cast<int64_t>(q_len) * (num_heads / num_kv_heads) > 16;
+}
+
 // Workspace: [header][ml: slots x 2 floats][acc: slots x head_dim floats], each
 // region 256-byte aligned. Slots cover both partial layouts: rows x max_parts for
 // the partition kernels, and pieces x UG x RT for stream-K decode, where pieces
@@ -237,6 +247,17 @@ Layout workspace_layout(int batch, int q_len, int num_heads, int num_kv_heads, i
   const int64_t pf_groups = prefill_sk_groups(batch, q_len, num_heads, num_kv_heads, head_dim,
                                               max_context, kPfSkMaxGroups);
   if (2 * pf_groups * kPfRows > L.slots) L.slots = 2 * pf_groups * kPfRows;
+  // The any-layout prefill kernel's shares: up to kPaReserve bytes, which leave a call that
+  // fits the no-allocation scratch without them inside it.
+  if (prefill_any_ok(batch, q_len, num_heads, num_kv_heads, head_dim)) {
+    const int64_t rows = static_cast<int64_t>(q_len) * (num_heads / num_kv_heads);
+    const int64_t tasks = (rows + kPfRows - 1) / kPfRows * num_kv_heads * batch;
+    const int64_t pairs = std::max<int64_t>(1, ceil_div(ceil_div(max_context, kPfStep), 2));
+    const int64_t row_bytes = static_cast<int64_t>(pa_capacity(head_dim) + 2) * sizeof(float);
+    const int64_t want = std::min<int64_t>(kPfSkMaxGroups, tasks * pairs) * 2 * kPfRows * row_bytes;
+    const int64_t have = std::min<int64_t>(want, kPaReserve) / ((head_dim + 2) * sizeof(float));
+    if (tasks <= kPaSkMaxTasks && have > L.slots) L.slots = have;
+  }
   // The header's prefix area: a stream-K decode's tiles per sequence (batch + 1 words), or a
   // stream-K prefill's task offsets and head size for its fold launch (tasks + 2).
   size_t prefix_words = static_cast<size_t>(batch) + 1;
@@ -849,6 +870,87 @@ bool prefill_preferred(int batch, int q_len, int num_heads, int num_kv_heads) {
   return 100 * ((rows + 15) / 16) * pairs > kPrefillSplitPct * cus * rounds;
 }
 
+// The any-layout prefill launch: its stream-K shares (0: one task per workgroup) and where the
+// shares' task offsets and partials sit in the workspace, which is the size the other kernels
+// of this geometry need (so that a call with its own workspace and the no-allocation entry
+// split the work alike): as many shares as fit there, at most one workgroup per CU.
+struct PaPlan {
+  int64_t groups = 0;
+  int head = 0;
+  int64_t cost_ns = 0;
+  size_t ml_offset = 0;
+  size_t acc_offset = 0;
+};
+
+PaPlan prefill_any_plan(int batch, int q_len, int num_heads, int num_kv_heads, int head_dim,
+                        int max_context, int q_dtype) {
+  PaPlan plan;
+  const int64_t rows = static_cast<int64_t>(q_len) * (num_heads / num_kv_heads);
+  const int64_t tasks = (rows + kPfRows - 1) / kPfRows * num_kv_heads * batch;
+  const int DP = pa_capacity(head_dim);
+  // A key-step pair of a 128-row task on one CU (17.5 us in fp32 at 128 dims, 3 us in 16 bits)
+  // and the fixed cost of a launch, more with shares (their second task starts, the partials
+  // and the fold): fitted on chunks of 64 to 4096 rows per KV head over 64 to 8192 keys.
+  const int64_t unit = (q_dtype == MSATTN_F32 ? 137 : 24) * DP;
+  const int64_t kSkFixed = q_dtype == MSATTN_F32 ? 35000 : 20000;
+  constexpr int64_t kOneFixed = 15000, kHeadNs = 6000;
+  const int64_t cus = device_cus();
+  const int64_t P = std::max<int64_t>(1, ceil_div(ceil_div(max_context, kPfStep), 2));
+  plan.cost_ns = (tasks + cus - 1) / cus * P * unit + kOneFixed;
+  if (tasks > kPaSkMaxTasks) return plan;
+  const Layout L = workspace_layout(batch, q_len, num_heads, num_kv_heads, head_dim, max_context);
+  const size_t ml_at = round256(sizeof(int) * (kHdrPrefix + static_cast<size_t>(tasks) + 2));
+  const size_t per_share = static_cast<size_t>(2) * kPfRows * (2 + DP) * sizeof(float);
+  const size_t total = L.total();
+  if (total < ml_at + 256 + per_share) return plan;
+  int64_t G = std::min<int64_t>({cus, kPfSkMaxGroups, tasks * P,
+                                 static_cast<int64_t>((total - ml_at - 256) / per_share)});
+  if (G >= kXcds) G = G / kXcds * kXcds;
+  if (G < 2) return plan;
+  const int64_t sk_cost = (tasks * P + G - 1) / G * unit + kSkFixed;
+  if (sk_cost >= plan.cost_ns) return plan;
+  plan.cost_ns = sk_cost;
+  plan.groups = G;
+  plan.head = static_cast<int>(std::min<int64_t>(kPfSkHead, kHeadNs / unit));
+  plan.ml_offset = ml_at;
+  plan.acc_offset = ml_at + round256(static_cast<size_t>(2 * G * kPfRows) * 2 * sizeof(float));
+  return plan;
+}
+
+// Whether query, cache rows and output all take the any-layout kernel's vector accesses.
+bool prefill_any_vec(const void* query, const void* out, int head_dim, bool rows16) {
+  return head_dim % 8 == 0 && rows16 && aligned(query, 16) && aligned(out, 16);
+}
+
+// Whether the any-layout kernel is the faster one for a chunk: its plan's cost against that of
+// the kernel the chunk takes otherwise. The partition kernel (an fp32 query at head_dim 64 or
+// 128) costs about 1.87 ns a 16-row, 16-key tile at 128 dims, 1.4 times that over a narrower
+// cache (913 us for 2 x 512 queries of H28/KVH4 over 4.6k keys), the generic kernel 2.45 ns
+// an 8-row, 16-key tile at 96 dims (182 us for 256 queries of H24/KVH8 over 1.8k keys); the
+// any-layout kernel takes those in 580 and 30 us, and where they hold few tiles (one sequence
+// of 49 queries, H14/KVH2/D128, 2000 keys: 30 against 88 us) it idles most CUs and loses.
+// Element loads double a step. Within 15 % the two measured level. Up to 96 rows per KV head, where its 128-row blocks are mostly
+// padding and the fit is coarse, it has to win twofold.
+bool prefill_any_preferred(int batch, int q_len, int num_heads, int num_kv_heads, int head_dim,
+                           int max_context, int q_dtype, int kv_dtype, bool mfma_decode, bool vec) {
+  const int64_t rows = static_cast<int64_t>(q_len) * (num_heads / num_kv_heads);
+  const int64_t pairs = static_cast<int64_t>(num_kv_heads) * batch;
+  const int64_t key_tiles = std::max<int64_t>(1, ceil_div(max_context, 16));
+  double old_ns;
+  if (mfma_decode)
+    old_ns = 10000.0 + 1.87 / 128 * head_dim * (kv_dtype == MSATTN_F32 ? 1.0 : 1.4) *
+                           static_cast<double>((rows + 15) / 16 * pairs) * key_tiles;
+  else
+    old_ns = 20000.0 + 2.45 / 96 * head_dim * (q_dtype == MSATTN_F32 ? 1.3 : 1.0) *
+                           static_cast<double>((rows + 7) / 8 * pairs) * key_tiles;
+  const double most = (rows > 96 ? 0.85 : 0.5) * old_ns;
+  if (most < 15000.0) return false;  // (less than the any-layout kernel's fixed cost)
+  const PaPlan plan = prefill_any_plan(batch, q_len, num_heads, num_kv_heads, head_dim, max_context,
+                                       q_dtype);
+  const double new_ns = vec ? plan.cost_ns : 2.0 * plan.cost_ns;
+  return new_ns < most;
+}
+
 // The route of msattn_paged_attention (and of the no-allocation entry point, whose
 // workspace is its scratch): the prefill kernel when it can run and the cost model
 // prefers it, or when the partition layout does not fit the workspace (the prefill
@@ -862,10 +964,18 @@ int choose_route(const void* query, const void* out, const void* k_cache, const 
                                    cache_head_stride, head_dim, kv_dtype);
   const Layout L = workspace_layout(batch, q_len, num_heads, num_kv_heads, head_dim, max_context);
   const bool fits = workspace_bytes >= L.total();
-  if (prefill_kernel_ok(query, out, cache_slot_stride, rows16, batch, q_len, num_heads,
-                        num_kv_heads, head_dim, block_size, q_dtype, kv_dtype) &&
-      (!fits || prefill_preferred(batch, q_len, num_heads, num_kv_heads)))
+  const bool copying = prefill_kernel_ok(query, out, cache_slot_stride, rows16, batch, q_len,
+                                         num_heads, num_kv_heads, head_dim, block_size, q_dtype,
+                                         kv_dtype);
+  if (copying && (!fits || prefill_preferred(batch, q_len, num_heads, num_kv_heads)))
     return MSATTN_ROUTE_PREFILL;
+  if (!copying && fits && prefill_any_ok(batch, q_len, num_heads, num_kv_heads, head_dim) &&
+      prefill_any_preferred(batch, q_len, num_heads, num_kv_heads, head_dim, max_context, q_dtype,
+                            kv_dtype,
+                            mfma_decode_route_ok(query, q_dtype, kv_dtype, head_dim, block_size,
+                                                 cache_slot_stride, rows16),
+                            prefill_any_vec(query, out, head_dim, rows16)))
+    return MSATTN_ROUTE_PREFILL_ANY;
   const PartialsPlan pl =
       plan_partials(query, q_dtype, kv_dtype, head_dim, block_size, cache_slot_stride, rows16,
                     batch, q_len, num_heads, num_kv_heads, max_context, true, 0);
@@ -890,9 +1000,11 @@ int attention_impl(const void* query, const void* k_cache, const void* v_cache,
   if (!dtype_ok(q_dtype) || !aligned(out, dtype_bytes(q_dtype))) return MSATTN_ERR_INVALID_ARG;
   if (!geometry_ok(batch, q_len, num_heads, num_kv_heads, head_dim, max_context))
     return MSATTN_ERR_INVALID_ARG;
-  if (choose_route(query, out, k_cache, v_cache, cache_block_stride, cache_slot_stride,
-                   cache_head_stride, batch, q_len, num_heads, num_kv_heads, head_dim, block_size,
-                   max_context, q_dtype, kv_dtype, workspace_bytes) == MSATTN_ROUTE_PREFILL) {
+  const int route = choose_route(query, out, k_cache, v_cache, cache_block_stride,
+                                 cache_slot_stride, cache_head_stride, batch, q_len, num_heads,
+                                 num_kv_heads, head_dim, block_size, max_context, q_dtype, kv_dtype,
+                                 workspace_bytes);
+  if (route == MSATTN_ROUTE_PREFILL || route == MSATTN_ROUTE_PREFILL_ANY) {
     if (!query || !block_table || !context_lens || !workspace) return MSATTN_ERR_INVALID_ARG;
     if (!std::isfinite(scale)) return MSATTN_ERR_INVALID_ARG;
     const int rc = check_cache_args(k_cache, v_cache, cache_block_stride, cache_slot_stride,
@@ -929,6 +1041,44 @@ int attention_impl(const void* query, const void* k_cache, const void* v_cache,
     const int64_t tasks = static_cast<int64_t>(pp.rblocks) * num_kv_heads * batch;
     if (tasks >= (int64_t(1) << 31) - kXcds) return MSATTN_ERR_UNSUPPORTED;
     pp.xcd_per = static_cast<int>((tasks + kXcds - 1) / kXcds);
+    bool sup = false;
+    const hipStream_t st = static_cast<hipStream_t>(stream);
+    if (route == MSATTN_ROUTE_PREFILL_ANY) {
+      if (!dtype_ok(kv_dtype) || q_dtype == MSATTN_FP8_E4M3 || !aligned(workspace, 16) ||
+          !aligned(query, dtype_bytes(q_dtype)))
+        return MSATTN_ERR_INVALID_ARG;
+      const bool rows16 = cache_rows16(k_cache, v_cache, cache_block_stride, cache_slot_stride,
+                                       cache_head_stride, head_dim, kv_dtype);
+      pp.head_dim = head_dim;
+      pp.vec = prefill_any_vec(query, out, head_dim, rows16) ? 1 : 0;
+      // A scale of zero weighs every visible key alike; a tiny one does the same and keeps
+      // the masked scores infinite.
+      if (scale == 0.0f) pp.scale_log2 = 1e-30f;
+      char* ws = static_cast<char*>(workspace);
+      pp.hdr = reinterpret_cast<int*>(ws);
+      pp.ntasks = static_cast<int>(tasks);
+      const PaPlan plan = prefill_any_plan(batch, q_len, num_heads, num_kv_heads, head_dim,
+                                           max_context, q_dtype);
+      if (plan.groups > 0) {
+        pp.sk_groups = static_cast<int>(plan.groups);
+        pp.sk_head = plan.head;
+        pp.sk_ml = reinterpret_cast<float*>(ws + plan.ml_offset);
+        pp.sk_acc = reinterpret_cast<float*>(ws + plan.acc_offset);
+        pp.sk_pre = pp.hdr + kHdrPrefix;
+      }
+      const auto by_cache = [&](auto t) {
+        using T = decltype(t);
+        switch (kv_dtype) {
+          case MSATTN_F32: return launch_prefill_any<T, float>(pp, st);
+          case MSATTN_F16: return launch_prefill_any<T, _Float16>(pp, st);
+          case MSATTN_BF16: return launch_prefill_any<T, bf16_t>(pp, st);
+          default: return launch_prefill_any<T, fp8_t>(pp, st);
+        }
+      };
+      return hip_status(q_dtype == MSATTN_F32   ? by_cache(float{})
+                        : q_dtype == MSATTN_F16 ? by_cache(_Float16{})
+                                                : by_cache(bf16_t{}));
+    }
     // Stream-K scheduling where the cost model prefers it (prefill_sk_plan): one workgroup
     // per CU, each taking an equal share of all tasks' key-step pairs; a task split
     // between shares is merged by the fold launch that follows (the work list's task
@@ -944,8 +1094,6 @@ int attention_impl(const void* query, const void* k_cache, const void* v_cache,
       pp.sk_acc = reinterpret_cast<float*>(ws + sk.acc_offset);
       pp.sk_pre = reinterpret_cast<int*>(ws) + kHdrPrefix;
     }
-    bool sup = false;
-    const hipStream_t st = static_cast<hipStream_t>(stream);
     const hipError_t e = with_mfma_types(q_dtype, kv_dtype, [&](auto t, auto kt) {
       return launch_prefill_mfma<decltype(t), decltype(kt)>(pp, head_dim, st, &sup);
     });

@@ -223,6 +223,13 @@ struct PrefillParams {
   float* sk_acc;      // [2 * sk_groups][kPfRows][D]
   int* sk_pre;        // [ntasks + 2]: the work list's task offsets and its head size,
                       // written by workgroup 0
+  // The any-layout kernel (prefill_any.h): the row's head size (its kernels are compiled for
+  // the next capacity), whether query, cache rows and output all take vector accesses, the
+  // workspace header, and the work list's head size.
+  int head_dim;
+  int vec;
+  int* hdr;
+  int sk_head;
 };
 
 // Largest task count of a stream-K prefill launch (its work-list prefix sums sit in LDS).

@@ -1,0 +1,126 @@
+"""The any-layout chunked-prefill kernel (csrc/prefill_any.h) against the float64 oracle.
+
+Bars, as the largest error over the largest output: the result's rounding to 16 bits is at
+most half a unit in the last place (2^-9 in bf16, 2^-12 in fp16, relative to the value), and
+everything before it is held to at least 2^-16, so twice the rounding: 2^-8 and 2^-11 (plus
+2^-14 for the weights' split in fp16). In fp32 the sums run over head_dim products and up to
+2100 keys, each within 2^-24 of its terms and random in sign: 64 * 2^-24 covers four standard
+deviations of sqrt(256) roundings twice.
+"""
+import numpy as np
+import pytest
+import torch
+
+from miniserve_amd import _native as nat
+from miniserve_amd import kernel_route, paged_attention
+from oracle import dense
+
+pytestmark = pytest.mark.gpu
+
+F32, F16, BF16, FP8 = torch.float32, torch.float16, torch.bfloat16, torch.float8_e4m3fn
+BAR = {F32: 64 * 2.0 ** -24, F16: 2.0 ** -11 + 2.0 ** -14, BF16: 2.0 ** -8}
+ROUTE = "prefill any-layout"
+
+
+def make(H, KVH, D, lens, q_len, q_dtype, kv_dtype, bs, seed, pad=0):
+    g = torch.Generator().manual_seed(seed)
+    counts = [max(1, -(-L // bs)) for L in lens]
+    pool = sum(counts) + 3
+    perm = torch.randperm(pool, generator=g)
+    # a table of 2^17 tokens: at that capacity the cost model takes this kernel for the chunks
+    # below (an fp32 one with few full row blocks stays on the partition kernel)
+    table = torch.zeros(len(lens), (1 << 17) // bs, dtype=torch.int32)
+    at = 0
+    for b, c in enumerate(counts):
+        table[b, :c] = perm[at:at + c]
+        at += c
+    q = torch.randn(len(lens), q_len, H, D, generator=g).to(q_dtype)
+    caches = []
+    for _ in range(2):
+        c = torch.zeros(pool, bs, KVH, D + pad, dtype=torch.float32)
+        c[..., :D] = torch.randn(pool, bs, KVH, D, generator=g)
+        caches.append(c.to(kv_dtype))
+    return q, caches[0], caches[1], table
+
+
+def check(device, q, kc, vc, table, lens, D, *, causal=True, window=None, scale=None):
+    qd, kd, vd, td = (x.to(device) for x in (q, kc, vc, table))
+    kd, vd = kd[..., :D], vd[..., :D]
+    ln = torch.tensor(lens, dtype=torch.int32, device=device)
+    assert kernel_route(qd, kd, td) == ROUTE
+    cap = table.shape[1] * kc.shape[1]
+    ws = torch.zeros(nat.lib().msattn_workspace_bytes(*q.shape[:2], q.shape[2], kc.shape[2], D, cap),
+                     dtype=torch.uint8, device=device)
+    outs = [paged_attention(qd, kd, vd, td, ln, causal=causal, window=window, scale=scale,
+                            workspace=ws) for _ in range(2)]
+    torch.cuda.synchronize()
+    assert torch.equal(outs[0], outs[1])
+    assert not ws[:(64 + 4096) * 4].view(torch.int32)[64:].any(), "tickets not at zero"
+    ref = dense.paged_attention_f64(q, kc[..., :D], vc[..., :D], table.long(), lens, causal=causal,
+                                    window=window, kv_cast=True,
+                                    **({} if scale is None else {"scale": scale}))
+    o = outs[0].double().cpu().numpy()
+    err = float(np.abs(o - ref).max() / max(np.abs(ref).max(), 1e-30))
+    print(f"[case] err {err:.2e}", flush=True)
+    assert err < BAR[q.dtype]
+    return outs[0]
+
+
+@pytest.mark.parametrize("q_dtype,kv_dtype,D", [
+    (q, kv, D) for q, kv in ((F32, F32), (BF16, BF16), (F16, F16), (F16, FP8), (BF16, F32))
+    for D in (30, 32, 40, 64, 80, 96, 112, 128, 160, 192, 200, 256)
+    if q == F32 or D not in (64, 128)])  # (those are the copying kernel's)
+def test_head_sizes(device, q_dtype, kv_dtype, D):
+    """Every compiled capacity at its size, below it and off 8-element rows: 381 rows per KV
+    head (two blocks and 125 rows) and a context that ends inside a page, one shorter than the
+    chunk, and one without keys."""
+    lens = [300, 20, 0, 127]
+    print(f"[case] D={D} {q_dtype}/{kv_dtype}", flush=True)
+    q, kc, vc, table = make(3, 1, D, lens, 127, q_dtype, kv_dtype, 16, D)
+    out = check(device, q, kc, vc, table, lens, D)
+    assert not out[2].any() and not out[1, :107].any()  # rows that see no key
+
+
+@pytest.mark.parametrize("q_dtype,kv_dtype", [(F32, BF16), (F32, F16), (F32, FP8), (F16, BF16),
+                                              (BF16, F16)])
+@pytest.mark.parametrize("H,KVH,D,bs,pad", [(8, 2, 128, 16, 0), (4, 4, 64, 24, 0), (6, 2, 96, 7, 0),
+                                            (8, 1, 64, 16, 3)])
+def test_layouts(device, q_dtype, kv_dtype, H, KVH, D, bs, pad):
+    """Type pairs, pages of 24 and 7 tokens, rows padded off 16-byte boundaries; windows and
+    non-causal chunks; a table with holes."""
+    q_len, lens = 130, [500, 131]
+    print(f"[case] {q_dtype}/{kv_dtype} H={H}/{KVH} D={D} bs={bs} pad={pad}", flush=True)
+    q, kc, vc, table = make(H, KVH, D, lens, q_len, q_dtype, kv_dtype, bs, 5, pad)
+    check(device, q, kc, vc, table, lens, D)
+    check(device, q, kc, vc, table, lens, D, window=70)
+    check(device, q, kc, vc, table, lens, D, causal=False, scale=-0.3)
+    table[0, 1] = -1
+    table[0, 9] = 10 ** 6
+    holed = paged_attention(q.to(device), kc.to(device)[..., :D], vc.to(device)[..., :D],
+                            table.to(device), lens)
+    keep = torch.ones(lens[0], dtype=torch.bool)
+    for pg in (1, 9):
+        keep[pg * bs:(pg + 1) * bs] = False
+    pages = table[0].clamp(0, kc.shape[0] - 1).long()
+    flat = [c[..., :D][pages].flatten(0, 1)[:lens[0]].to(q_dtype).double() for c in (kc, vc)]
+    k, v = (x.repeat_interleave(H // KVH, 1) for x in flat)
+    s = torch.einsum("qhd,khd->hqk", q[0].double(), k) / D ** 0.5
+    pos = torch.arange(lens[0])
+    seen = (pos[None, :] <= lens[0] - q_len + torch.arange(q_len)[:, None]) & keep[None, :]
+    ref = torch.einsum("hqk,khd->qhd", s.masked_fill(~seen, -torch.inf).softmax(-1), v)
+    err = (holed[0].double().cpu() - ref).abs().max() / ref.abs().max()
+    assert err < BAR[q_dtype]
+
+
+@pytest.mark.parametrize("H,KVH,D,q_len,lens,q_dtype", [
+    (2, 1, 128, 200, [2100], F32),          # four tasks over every CU: shares of a pair
+    (8, 8, 64, 380, [1900, 400, 700], F32),  # uneven tasks, three row blocks each
+    (6, 2, 96, 256, [2000], BF16),
+    (4, 1, 256, 64, [1500, 90], F16),
+    (24, 8, 80, 300, [1000, 301], BF16),
+])
+def test_shares(device, H, KVH, D, q_len, lens, q_dtype):
+    """Few tasks over long contexts: the work list split between workgroups and folded."""
+    print(f"[case] shares H={H}/{KVH} D={D} q_len={q_len} {q_dtype}", flush=True)
+    q, kc, vc, table = make(H, KVH, D, lens, q_len, q_dtype, q_dtype, 16, q_len)
+    check(device, q, kc, vc, table, lens, D)
