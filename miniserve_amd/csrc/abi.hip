@@ -191,7 +191,8 @@ constexpr int kSkMinChunk = MSATTN_SK_MIN_CHUNK;  // stream-K: smallest chunk (t
 int mfma_rows_per_tile(int rows_per_kvh) { return rows_per_kvh >= 16 ? 16 : next_pow2(rows_per_kvh); }
 
 // A multi-token query of more than 16 rows per KV head that the copying prefill kernel cannot
-// take may run on the any-layout prefill kernel (prefill_any.h): its geometry.
+// take may run on the any-layout prefill kernel (prefill_any.h): its geometry. (Decodes do not:
+// at other head sizes the generic kernel measured 1.3-1.9 times faster on 16-bit caches.)
 constexpr int64_t kPaReserve = 40 << 20;  // bytes of share partials a workspace reserves
 
 bool prefill_any_ok(int batch, int q_len, int num_heads, int num_kv_heads, int head_dim) {
@@ -691,13 +692,14 @@ int partials_impl(const void* query, const void* k_cache, const void* v_cache,
         p.max_parts = np;
       }
     }
-    // Few (sequence, KV head, row tile) triples over long contexts: when partitions that
-    // give about one workgroup per CU would hold kPartWide tokens or more, and the launch
-    // stays within 1.5 workgroups per CU, the partition kernel's wide shape (8 waves, two
-    // per SIMD) over kPartWide-token partitions. Its
-    // two waves per SIMD fill each other's waits (C5-decode: 24.1 -> 22.6 us); shorter
-    // wide partitions, and wide workgroups two to a CU, measured slower than the regular
-    // shape.
+    // Few (sequence, KV head, row tile) triples over long contexts: when kPartWide-token
+    // partitions give about a workgroup per CU or more (the last of them possibly short), and
+    // the launch stays within 1.5 workgroups per CU, the partition kernel's wide shape (8
+    // waves, two per SIMD). Its two waves per SIMD fill each other's waits (C5-decode: 24.1 ->
+    // 22.6 us). A table that ends inside the last partition counts: 16 x H28/KVH4/D128 at 3500
+    // tokens 30.0 -> 25.9 us (fp8 cache 26.0 -> 21.1), 12 x 5100 31.8 -> 27.3, 24 x 1040
+    // 22.4 -> 20.7, 8 x H32/KVH8 at 3500 27.3 -> 24.9, level at 3936 and 5 x 5100. Shorter
+    // wide partitions, and wide workgroups two to a CU, measured slower than the regular shape.
     if (kWideRoute && q_len == 1 && (RT == 4 || RT == 8) && q_dtype != MSATTN_F32 &&
         kv_dtype != MSATTN_F32) {
       const int64_t triples = static_cast<int64_t>(batch) * num_kv_heads * p.rtiles;
@@ -709,7 +711,7 @@ int partials_impl(const void* query, const void* k_cache, const void* v_cache,
       // (5-10 % faster on H32/KVH8 decodes of 6-20 workgroups per CU); at 8 rows per tile,
       // at head_dim 64 and over a 16-bit cache the cap stands (7-18 % slower without it).
       const bool uncapped = kWideFp8Uncapped && kv_fp8 && RT == 4 && head_dim == 128;
-      if (static_cast<int64_t>(max_context) >= np * kPartWide &&
+      if (ceil_div(max_context, kPartWide) >= np &&
           (uncapped || 100 * launched <= static_cast<int64_t>(kWideMaxPct) * want)) {
         p.part = kPartWide;
         p.max_parts = ceil_div(max_context, kPartWide);
