@@ -139,6 +139,25 @@ int msattn_paged_attention(const void* query, const void* k_cache, const void* v
                            float scale, int q_dtype, int kv_dtype, void* stream);
 
 /*
+ * msattn_paged_attention over a query whose batch, token and head strides (elements, at
+ * least 0) are given and whose head dim is contiguous: a chunked prefill then reads a view,
+ * such as a model's transposed projections (miniserve/model_runner.py:62-67), without a copy
+ * made of it first. Same results. Calls that the two prefill kernels do not take return
+ * MSATTN_ERR_UNSUPPORTED and launch nothing (the copying kernel needs 16-byte multiples).
+ * The output must not overlap the query.
+ */
+int msattn_paged_attention_strided(const void* query, int64_t q_batch_stride,
+                                   int64_t q_token_stride, int64_t q_head_stride,
+                                   const void* k_cache, const void* v_cache,
+                                   int64_t cache_block_stride, int64_t cache_slot_stride,
+                                   int64_t cache_head_stride, const int32_t* block_table,
+                                   const int32_t* context_lens, void* out, void* workspace,
+                                   size_t workspace_bytes, int batch, int q_len, int num_heads,
+                                   int num_kv_heads, int head_dim, int block_size, int num_blocks,
+                                   int table_width, int max_context, int causal, int window,
+                                   float scale, int q_dtype, int kv_dtype, void* stream);
+
+/*
  * msattn_paged_attention without the workspace arguments, for callers that cannot
  * allocate (code under hipGraph capture that must not call hipMalloc, tight serving
  * loops, harnesses that forbid allocation). No counterpart in the reference, whose
@@ -280,6 +299,19 @@ int msattn_write_kv(void* k_cache, void* v_cache, int64_t cache_block_stride,
                     int batch, int tokens, int num_kv_heads, int head_dim, int block_size,
                     int num_blocks, int table_width, int src_dtype, int kv_dtype,
                     void* stream);
+
+/*
+ * msattn_write_kv from sources with the given batch, token and head strides (elements, at
+ * least 0), head dim contiguous; the same writes. The sources must not overlap the caches.
+ */
+int msattn_write_kv_strided(void* k_cache, void* v_cache, int64_t cache_block_stride,
+                            int64_t cache_slot_stride, int64_t cache_head_stride, const void* k,
+                            int64_t k_batch_stride, int64_t k_token_stride, int64_t k_head_stride,
+                            const void* v, int64_t v_batch_stride, int64_t v_token_stride,
+                            int64_t v_head_stride, const int32_t* block_table,
+                            const int32_t* starts, int batch, int tokens, int num_kv_heads,
+                            int head_dim, int block_size, int num_blocks, int table_width,
+                            int src_dtype, int kv_dtype, void* stream);
 
 /*
  * Decode with the new token appended: msattn_write_kv of k_new / v_new at position

@@ -64,6 +64,14 @@ def apply_rope(q: torch.Tensor, k: torch.Tensor | None, cos: torch.Tensor, sin: 
     return q_rot, k_rot
 
 
+def _readable_in_place(t: torch.Tensor, *written: torch.Tensor | None) -> bool:
+    """Whether a kernel may read `t` [batch, tokens, heads, dim] through its strides: rows of
+    contiguous dims, in memory that none of the tensors the call writes shares."""
+    base = t.untyped_storage().data_ptr()
+    return t.stride(3) == 1 and t.numel() > 0 and not t.is_neg() and \
+        all(w is None or w.untyped_storage().data_ptr() != base for w in written)
+
+
 def _require_gpu(t: torch.Tensor, what: str) -> None:
     if t.device.type != "cuda":
         raise RuntimeError(
@@ -242,6 +250,17 @@ class PagedAttention:
         if starts.numel() < B:
             raise ValueError("start needs one entry per batch row")
         starts = starts.contiguous()
+        if not (k.is_contiguous() and v.is_contiguous()) and \
+                _readable_in_place(k, k_cache, v_cache) and _readable_in_place(v, k_cache, v_cache):
+            # views, such as a model's transposed projections, are read where they lie
+            status = nat.lib().msattn_write_kv_strided(
+                k_cache.data_ptr(), v_cache.data_ptr(), k_cache.stride(0), k_cache.stride(1),
+                k_cache.stride(2), k.data_ptr(), *k.stride()[:3], v.data_ptr(), *v.stride()[:3],
+                table.data_ptr(), starts.data_ptr(), B, T, KVH, D, k_cache.shape[1],
+                k_cache.shape[0], table.shape[1], nat.dtype_code(k.dtype),
+                nat.dtype_code(k_cache.dtype), nat.stream_handle(dev))
+            nat.check("msattn_write_kv_strided", status)
+            return
         kc = k.contiguous()
         vc = v.contiguous()
         status = nat.lib().msattn_write_kv(
@@ -370,7 +389,6 @@ def paged_attention(query: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.T
     if window is not None and window <= 0:
         raise ValueError("window must be positive")
     dev = query.device
-    q = query.contiguous()
     table = block_table_i32(block_table, dev)
     if table.shape[0] != B:
         raise ValueError(f"block_table has {table.shape[0]} rows for a batch of {B}")
@@ -402,8 +420,21 @@ def paged_attention(query: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.T
     if workspace is None or workspace.numel() * workspace.element_size() < ws_bytes:
         # zeroed: the in-kernel merge's tickets must start at zero (calls leave them so)
         workspace = _workspace(dev, ws_bytes)
+    in_place = q_len > 1 and not prefix_pages and rope is None and not query.is_contiguous() and \
+        _readable_in_place(query, out)
     if out is None:
         out = torch.empty((B, q_len, H, D), dtype=query.dtype, device=dev)
+    if in_place:  # a chunked prefill reads a view of the query where it lies
+        status = L.msattn_paged_attention_strided(
+            query.data_ptr(), *query.stride()[:3], k_cache.data_ptr(), v_cache.data_ptr(),
+            k_cache.stride(0), k_cache.stride(1), k_cache.stride(2), table.data_ptr(),
+            lens.data_ptr(), out.data_ptr(), workspace.data_ptr(), ws_bytes, B, q_len, H, KVH, D,
+            bs, nb, W, max_context, 1 if causal else 0, int(window or 0), float(scale), qcode,
+            kvcode, nat.stream_handle(dev))
+        if status != nat.ERR_UNSUPPORTED:
+            nat.check("msattn_paged_attention_strided", status)
+            return out
+    q = query.contiguous()
     args = (q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), k_cache.stride(0),
             k_cache.stride(1), k_cache.stride(2), table.data_ptr(), lens.data_ptr(),
             out.data_ptr(), workspace.data_ptr(), ws_bytes, B, q_len, H, KVH, D, bs, nb, W,

@@ -68,7 +68,7 @@ int write_kv_impl(void* k_cache, void* v_cache, int64_t cache_block_stride,
                   const void* v, const int32_t* block_table, const int32_t* starts,
                   int start_offset, int batch, int tokens, int num_kv_heads, int head_dim,
                   int block_size, int num_blocks, int table_width, int src_dtype, int kv_dtype,
-                  void* stream);
+                  void* stream, const int64_t* src_strides = nullptr);
 #ifndef MSATTN_WIDE_ROUTE
 #define MSATTN_WIDE_ROUTE 1
 #endif
@@ -988,7 +988,9 @@ int choose_route(const void* query, const void* out, const void* k_cache, const 
 
 // msattn_paged_attention's body. `prefill_needs_ws`: whether the direct prefill route
 // checks the workspace size too (the workspace entry point's contract), although that
-// route does not touch it.
+// route does not touch it. `q_strides`: batch, token and head strides of a query that is not
+// contiguous, which the prefill kernels read in place; calls on other routes, and strides the
+// copying kernel's 16-byte loads cannot take, return MSATTN_ERR_UNSUPPORTED unlaunched.
 int attention_impl(const void* query, const void* k_cache, const void* v_cache,
                    int64_t cache_block_stride, int64_t cache_slot_stride,
                    int64_t cache_head_stride, const int32_t* block_table,
@@ -997,7 +999,8 @@ int attention_impl(const void* query, const void* k_cache, const void* v_cache,
                    int num_kv_heads, int head_dim, int block_size, int num_blocks,
                    int table_width, int max_context, int causal, int window, float scale,
                    int q_dtype, int kv_dtype, bool prefill_needs_ws, void* stream,
-                   const void* k_new = nullptr, const void* v_new = nullptr) {
+                   const void* k_new = nullptr, const void* v_new = nullptr,
+                   const int64_t* q_strides = nullptr) {
   if (!out) return MSATTN_ERR_INVALID_ARG;
   if (!dtype_ok(q_dtype) || !aligned(out, dtype_bytes(q_dtype))) return MSATTN_ERR_INVALID_ARG;
   if (!geometry_ok(batch, q_len, num_heads, num_kv_heads, head_dim, max_context))
@@ -1006,6 +1009,15 @@ int attention_impl(const void* query, const void* k_cache, const void* v_cache,
                                  cache_slot_stride, cache_head_stride, batch, q_len, num_heads,
                                  num_kv_heads, head_dim, block_size, max_context, q_dtype, kv_dtype,
                                  workspace_bytes);
+  const int64_t q_row = head_dim, q_tok = q_row * num_heads;
+  const int64_t dense_q[3] = {q_tok * q_len, q_tok, q_row};
+  const int64_t* const qs = q_strides != nullptr ? q_strides : dense_q;
+  const bool qs16 = (qs[0] * dtype_bytes(q_dtype)) % 16 == 0 &&
+                    (qs[1] * dtype_bytes(q_dtype)) % 16 == 0 &&
+                    (qs[2] * dtype_bytes(q_dtype)) % 16 == 0;
+  if (q_strides != nullptr && route != MSATTN_ROUTE_PREFILL_ANY &&
+      !(route == MSATTN_ROUTE_PREFILL && qs16))
+    return MSATTN_ERR_UNSUPPORTED;
   if (route == MSATTN_ROUTE_PREFILL || route == MSATTN_ROUTE_PREFILL_ANY) {
     if (!query || !block_table || !context_lens || !workspace) return MSATTN_ERR_INVALID_ARG;
     if (!std::isfinite(scale)) return MSATTN_ERR_INVALID_ARG;
@@ -1025,6 +1037,9 @@ int attention_impl(const void* query, const void* k_cache, const void* v_cache,
     pp.blk_stride = cache_block_stride;
     pp.slot_stride = cache_slot_stride;
     pp.head_stride = cache_head_stride;
+    pp.q_batch = qs[0];
+    pp.q_token = qs[1];
+    pp.q_head = qs[2];
     pp.batch = batch;
     pp.q_len = q_len;
     pp.H = num_heads;
@@ -1052,7 +1067,7 @@ int attention_impl(const void* query, const void* k_cache, const void* v_cache,
       const bool rows16 = cache_rows16(k_cache, v_cache, cache_block_stride, cache_slot_stride,
                                        cache_head_stride, head_dim, kv_dtype);
       pp.head_dim = head_dim;
-      pp.vec = prefill_any_vec(query, out, head_dim, rows16) ? 1 : 0;
+      pp.vec = prefill_any_vec(query, out, head_dim, rows16) && qs16 ? 1 : 0;
       // A scale of zero weighs every visible key alike; a tiny one does the same and keeps
       // the masked scores infinite.
       if (scale == 0.0f) pp.scale_log2 = 1e-30f;
@@ -1160,6 +1175,25 @@ int msattn_paged_attention(const void* query, const void* k_cache, const void* v
                         workspace_bytes, batch, q_len, num_heads, num_kv_heads, head_dim,
                         block_size, num_blocks, table_width, max_context, causal, window, scale,
                         q_dtype, kv_dtype, true, stream);
+}
+
+int msattn_paged_attention_strided(const void* query, int64_t q_batch_stride,
+                                   int64_t q_token_stride, int64_t q_head_stride,
+                                   const void* k_cache, const void* v_cache,
+                                   int64_t cache_block_stride, int64_t cache_slot_stride,
+                                   int64_t cache_head_stride, const int32_t* block_table,
+                                   const int32_t* context_lens, void* out, void* workspace,
+                                   size_t workspace_bytes, int batch, int q_len, int num_heads,
+                                   int num_kv_heads, int head_dim, int block_size, int num_blocks,
+                                   int table_width, int max_context, int causal, int window,
+                                   float scale, int q_dtype, int kv_dtype, void* stream) {
+  if (q_batch_stride < 0 || q_token_stride < 0 || q_head_stride < 0) return MSATTN_ERR_INVALID_ARG;
+  const int64_t strides[3] = {q_batch_stride, q_token_stride, q_head_stride};
+  return attention_impl(query, k_cache, v_cache, cache_block_stride, cache_slot_stride,
+                        cache_head_stride, block_table, context_lens, out, workspace,
+                        workspace_bytes, batch, q_len, num_heads, num_kv_heads, head_dim,
+                        block_size, num_blocks, table_width, max_context, causal, window, scale,
+                        q_dtype, kv_dtype, true, stream, nullptr, nullptr, strides);
 }
 
 int msattn_paged_attention_noalloc(const void* query, const void* k_cache, const void* v_cache,
@@ -1312,6 +1346,9 @@ int msattn_paged_attention_prefix(const void* query, const void* k_cache, const 
   pp.blk_stride = cache_block_stride;
   pp.slot_stride = cache_slot_stride;
   pp.head_stride = cache_head_stride;
+  pp.q_batch = 0;  // one virtual sequence, a token a row of the batch
+  pp.q_token = static_cast<int64_t>(num_heads) * head_dim;
+  pp.q_head = head_dim;
   pp.batch = 1;
   pp.q_len = batch;
   pp.H = num_heads;
@@ -1364,6 +1401,23 @@ int msattn_write_kv(void* k_cache, void* v_cache, int64_t cache_block_stride,
                        cache_head_stride, k, v, block_table, starts, 0, batch, tokens,
                        num_kv_heads, head_dim, block_size, num_blocks, table_width, src_dtype,
                        kv_dtype, stream);
+}
+
+int msattn_write_kv_strided(void* k_cache, void* v_cache, int64_t cache_block_stride,
+                            int64_t cache_slot_stride, int64_t cache_head_stride, const void* k,
+                            int64_t k_batch_stride, int64_t k_token_stride, int64_t k_head_stride,
+                            const void* v, int64_t v_batch_stride, int64_t v_token_stride,
+                            int64_t v_head_stride, const int32_t* block_table,
+                            const int32_t* starts, int batch, int tokens, int num_kv_heads,
+                            int head_dim, int block_size, int num_blocks, int table_width,
+                            int src_dtype, int kv_dtype, void* stream) {
+  const int64_t strides[6] = {k_batch_stride, k_token_stride, k_head_stride,
+                              v_batch_stride, v_token_stride, v_head_stride};
+  for (int64_t x : strides)
+    if (x < 0) return MSATTN_ERR_INVALID_ARG;
+  return write_kv_impl(k_cache, v_cache, cache_block_stride, cache_slot_stride, cache_head_stride, k,
+                       v, block_table, starts, 0, batch, tokens, num_kv_heads, head_dim, block_size,
+                       num_blocks, table_width, src_dtype, kv_dtype, stream, strides);
 }
 
 int msattn_paged_attention_append(const void* query, const void* k_new, const void* v_new,
@@ -1419,7 +1473,7 @@ int write_kv_impl(void* k_cache, void* v_cache, int64_t cache_block_stride,
                   const void* v, const int32_t* block_table, const int32_t* starts,
                   int start_offset, int batch, int tokens, int num_kv_heads, int head_dim,
                   int block_size, int num_blocks, int table_width, int src_dtype, int kv_dtype,
-                  void* stream) {
+                  void* stream, const int64_t* src_strides) {
   if (!k_cache || !v_cache || !k || !v || !block_table || !starts) return MSATTN_ERR_INVALID_ARG;
   if (batch <= 0 || tokens < 0 || num_kv_heads <= 0 || head_dim <= 0) return MSATTN_ERR_INVALID_ARG;
   if (block_size <= 0 || num_blocks <= 0 || table_width <= 0) return MSATTN_ERR_INVALID_ARG;
@@ -1441,6 +1495,12 @@ int write_kv_impl(void* k_cache, void* v_cache, int64_t cache_block_stride,
   p.blk_stride = cache_block_stride;
   p.slot_stride = cache_slot_stride;
   p.head_stride = cache_head_stride;
+  const int64_t row = head_dim, tok = row * num_kv_heads;
+  const int64_t dense[6] = {tok * tokens, tok, row, tok * tokens, tok, row};
+  for (int i = 0; i < 3; ++i) {
+    p.k_src[i] = (src_strides != nullptr ? src_strides : dense)[i];
+    p.v_src[i] = (src_strides != nullptr ? src_strides : dense)[3 + i];
+  }
   p.batch = batch;
   p.tokens = tokens;
   p.KVH = num_kv_heads;

@@ -18,6 +18,11 @@ __device__ __forceinline__ int64_t token_offset(const int32_t* table, int b, int
   return static_cast<int64_t>(phys) * blk_stride + static_cast<int64_t>(pos - pg * bs) * slot_stride;
 }
 
+// Element offset of (row b, token t, head h) in a source of strides s.
+__device__ __forceinline__ int64_t source_offset(const int64_t (&s)[3], int b, int t, int h) {
+  return b * s[0] + t * s[1] + h * s[2];
+}
+
 // write_kv: cache[table[b, pos/bs], pos%bs, h, d] = convert(src[b, t, h, d]),
 // pos = starts[b] + t (miniserve/attention.py:111-133). One thread per element.
 template <typename ST, typename DT>
@@ -35,8 +40,10 @@ __global__ __launch_bounds__(kOpsThreads) void write_kv_kernel(const WriteKVPara
                                      p.blk_stride, p.slot_stride);
     if (off < 0) continue;
     const int64_t dst = off + static_cast<int64_t>(h) * p.head_stride + d;
-    Elt<DT>::store(static_cast<DT*>(p.k_cache) + dst, Elt<ST>::load(static_cast<const ST*>(p.k) + idx));
-    Elt<DT>::store(static_cast<DT*>(p.v_cache) + dst, Elt<ST>::load(static_cast<const ST*>(p.v) + idx));
+    Elt<DT>::store(static_cast<DT*>(p.k_cache) + dst,
+                   Elt<ST>::load(static_cast<const ST*>(p.k) + source_offset(p.k_src, b, t, h) + d));
+    Elt<DT>::store(static_cast<DT*>(p.v_cache) + dst,
+                   Elt<ST>::load(static_cast<const ST*>(p.v) + source_offset(p.v_src, b, t, h) + d));
   }
 }
 
@@ -56,8 +63,8 @@ __global__ __launch_bounds__(kOpsThreads) void write_kv_copy_kernel(const WriteK
                                      p.blk_stride, p.slot_stride);
     if (off < 0) continue;
     const int64_t dst = off + static_cast<int64_t>(h) * p.head_stride + d;
-    static_cast<T*>(p.k_cache)[dst] = static_cast<const T*>(p.k)[idx];
-    static_cast<T*>(p.v_cache)[dst] = static_cast<const T*>(p.v)[idx];
+    static_cast<T*>(p.k_cache)[dst] = static_cast<const T*>(p.k)[source_offset(p.k_src, b, t, h) + d];
+    static_cast<T*>(p.v_cache)[dst] = static_cast<const T*>(p.v)[source_offset(p.v_src, b, t, h) + d];
   }
 }
 
@@ -86,11 +93,11 @@ __global__ __launch_bounds__(kOpsThreads) void write_kv_vec_kernel(const WriteKV
     const int64_t off = token_offset(p.table, b, p.starts[b] + p.start_offset + t, p.bs, p.W, p.num_blocks,
                                      p.blk_stride, p.slot_stride);
     if (off < 0) continue;
-    const int64_t src = idx * E;  // [b, t, h, c * E] of the contiguous source
     const int64_t dst = off + static_cast<int64_t>(h) * p.head_stride + static_cast<int64_t>(c) * E;
 #pragma unroll
     for (int which = 0; which < 2; ++which) {
-      const ST* sp = static_cast<const ST*>(which ? p.v : p.k) + src;
+      const ST* sp = static_cast<const ST*>(which ? p.v : p.k) +
+                     source_offset(which ? p.v_src : p.k_src, b, t, h) + c * E;
       DT* dp = static_cast<DT*>(which ? p.v_cache : p.k_cache) + dst;
       if constexpr (std::is_same<ST, DT>::value) {
         *reinterpret_cast<RawN<E * sizeof(ST)>*>(dp) =
@@ -116,12 +123,14 @@ static unsigned grid_for(int64_t total) {
 }
 
 // Whether the vector form with E elements per thread applies: head_dim a multiple of E,
-// the source (contiguous) on E source elements' alignment, the caches and their strides
-// on E cache elements' alignment.
+// the sources and their strides on E source elements' alignment, the caches and theirs on E
+// cache elements'.
 template <typename ST, typename DT, int E>
 static bool wkv_vec_ok(const WriteKVParams& p) {
   const uintptr_t sa = E * sizeof(ST), da = E * sizeof(DT);
   auto al = [](const void* q, uintptr_t a) { return reinterpret_cast<uintptr_t>(q) % a == 0; };
+  for (int i = 0; i < 3; ++i)
+    if (p.k_src[i] % E != 0 || p.v_src[i] % E != 0) return false;
   return p.D % E == 0 && al(p.k, sa) && al(p.v, sa) && al(p.k_cache, da) && al(p.v_cache, da) &&
          (p.blk_stride * sizeof(DT)) % da == 0 && (p.slot_stride * sizeof(DT)) % da == 0 &&
          (p.head_stride * sizeof(DT)) % da == 0;

@@ -336,7 +336,10 @@ __global__ __launch_bounds__(pa_groups(DP) * kPfGroupThreads) void prefill_any_k
     // The query row: B operand chunk j = dims (F32: 8 j + 4 hh .. + 3; else 16 j + 8 hh .. + 7).
     uint4 qb[JD];
     {
-      const T* qp = static_cast<const T*>(p.q) + (row_ok ? out_row() * D : 0);
+      const int i = row_ok ? row / p.G : 0;
+      const T* qp = static_cast<const T*>(p.q) +
+                    (row_ok ? b * p.q_batch + i * p.q_token + (kvh * p.G + (row - i * p.G)) * p.q_head
+                            : 0);
 #pragma unroll
       for (int j = 0; j < JD; ++j) {
         const int d0 = NE * (2 * j + hh);

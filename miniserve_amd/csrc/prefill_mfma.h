@@ -195,6 +195,7 @@ struct PrefillParams {
   const int32_t* lens;
   void* out;
   int64_t blk_stride, slot_stride, head_stride;
+  int64_t q_batch, q_token, q_head;  // query strides (elements)
   int batch, q_len, H, KVH, G;
   int bs, num_blocks, W, max_ctx;
   int causal, window;
@@ -489,8 +490,8 @@ __global__ __launch_bounds__(kPfThreads) void prefill_mfma_kernel(const PrefillP
   // it, each for half of every 8 keys or dims).
   const bool row_ok = row0 + w * WROWS + cc < p.rows_per_kvh;
   int lo_n = 0, hi_n = 0;
-  // Index of the lane's query row in the [tokens, heads] query / output arrays
-  // (recomputed where needed rather than held through the key loop).
+  // Index of the lane's query row in the [tokens, heads] output array (recomputed where
+  // needed rather than held through the key loop).
   auto out_row = [&]() {
     const int row = row0 + w * WROWS + cc;
     const int i = row / p.G;
@@ -530,11 +531,14 @@ __global__ __launch_bounds__(kPfThreads) void prefill_mfma_kernel(const PrefillP
   // The B operand Q^T of k-step j: the row's dims 16 j + 8 hh .. + 7.
   uint4 qb[JD];
   {
-    const T* qp = static_cast<const T*>(p.q);
+    const int row = row0 + w * WROWS + cc;
+    const int i = row / p.G;
+    const T* qp = static_cast<const T*>(p.q) + b * p.q_batch + i * p.q_token +
+                  (kvh * p.G + (row - i * p.G)) * p.q_head + 8 * hh;
 #pragma unroll
     for (int j = 0; j < JD; ++j) {
       qb[j] = make_uint4(0u, 0u, 0u, 0u);
-      if (row_ok) qb[j] = *reinterpret_cast<const uint4*>(qp + out_row() * D + 16 * j + 8 * hh);
+      if (row_ok) qb[j] = *reinterpret_cast<const uint4*>(qp + 16 * j);
     }
   }
 
