@@ -280,15 +280,23 @@ __device__ __forceinline__ PfTask pf_task(const PrefillParams& p, unsigned task)
   return t;
 }
 
-template <typename T, typename KT, int D, int RB, bool PX>
+// STEPWISE: an fp8 cache staged step by step (always so for an fp32 cache).
+template <typename T, typename KT, int D, int RB, bool PX, bool STEPWISE = false>
 __global__ __launch_bounds__(kPfThreads) void prefill_mfma_kernel(const PrefillParams p) {
   typedef Kv8<T, KT> KV;  // a cache of T, or of fp8 e4m3 / fp32 converted to T in registers
   typedef typename KV::raw_t raw_t;
   constexpr int EB = static_cast<int>(sizeof(KT));
   static_assert(D == 64 || D == 128, "prefill MFMA kernel handles head_dim 64 and 128");
-  // A cache of the query's type is copied into LDS by the load unit; other caches pass
-  // through registers, where they are converted.
-  constexpr bool DMA = MSATTN_PF_DMA && std::is_same<T, KT>::value;
+  // A cache of the query's type is copied into LDS by the load unit. An fp8 cache takes the
+  // same schedule, its rows passing through registers (8 or 16 of them), widened on the way: the
+  // loads go out where the copies would, the LDS writes before the iteration's barrier. 2 x 512
+  // queries over 4.6k keys, H28/KVH4/D128 fp16 over fp8: 106.6 -> 85.6 us (603 -> 746
+  // TFLOP/s; the step-by-step staging left both key groups in phase). Loads issued at the
+  // iteration's start instead: 89. STEPWISE keeps the step-by-step staging for the tasks of few
+  // steps (pf_stepwise), and an fp32 cache, whose rows would hold four times the registers,
+  // always takes it.
+  constexpr bool WIDEN = std::is_same<KT, fp8_t>::value && !STEPWISE;
+  constexpr bool DMA = MSATTN_PF_DMA && (std::is_same<T, KT>::value || WIDEN);
   constexpr int JD = D / 16;              // k-steps of S^T (16 dims each)
   constexpr int ND = D / 32;              // 32-dim tiles of O^T
   static_assert(16 * RB == 32, "one 32-row MFMA block per wave");
@@ -733,8 +741,8 @@ __global__ __launch_bounds__(kPfThreads) void prefill_mfma_kernel(const PrefillP
     // one chunk each) and the transposed V reads (8 rows, 32 bytes each) then fall on
     // distinct banks. Tokens past hi_all, below a window's first key, or on a page the table
     // does not map lie outside the tile's descriptor: their copies write zeros.
-    constexpr int CPRD = D / 8;        // 16-byte chunks per row
-    constexpr int RPI = kWave / CPRD;  // rows per copy instruction (4 or 8)
+    constexpr int CPRD = D * EB / 16;  // 16-byte chunks per row, as stored in the cache
+    constexpr int RPI = kWave / CPRD;  // rows per copy instruction (4 or 8; fp8 8 or 16)
     constexpr int NI = 16 / RPI;       // copy instructions per 16-row tile
     // Lane byte offsets of the reads, as one base XORed with a constant per k-step / dim
     // tile, so no register per j or t is held (slots are 256-byte aligned, rows 2 D
@@ -749,7 +757,8 @@ __global__ __launch_bounds__(kPfThreads) void prefill_mfma_kernel(const PrefillP
 #pragma unroll
     for (int j = 0; j < NI; ++j) {
       const int lr = RPI * j + lane / CPRD;
-      dvo[j] = static_cast<uint32_t>(lr * row_bytes + 16 * ((lane % CPRD) ^ pf_swz<D>(lr)));
+      dvo[j] = static_cast<uint32_t>(lr * row_bytes +
+                                     16 * (WIDEN ? lane % CPRD : (lane % CPRD) ^ pf_swz<D>(lr)));
     }
     // This wave's 16-row tile of a step (token rows 16 w ..): one descriptor for its K
     // rows and one for its V rows, and the offset that pushes rows below a window's first
@@ -805,9 +814,26 @@ __global__ __launch_bounds__(kPfThreads) void prefill_mfma_kernel(const PrefillP
       c.skip = static_cast<uint32_t>(skip * row_bytes);  // rows below wrap out of range
       return c;
     };
-    // Copy instruction j of the tile (RPI token rows) into the LDS slot dst.
-    auto copy_rows = [&](__amdgpu_buffer_rsrc_t r, uint32_t skip, uint16_t* dst, int j) {
-      lds_copy16(r, dst + (16 * w + RPI * j) * D, dvo[j] - skip);
+    // Copy instruction j of the tile (RPI token rows) into the LDS slot dst; from an fp8 cache,
+    // into held[j], which land() widens and writes to the slot.
+    uint4 k_held[WIDEN ? NI : 1], v_held[WIDEN ? NI : 1];
+    auto copy_rows = [&](__amdgpu_buffer_rsrc_t r, uint32_t skip, uint16_t* dst, uint4* held, int j) {
+      if constexpr (WIDEN) held[j] = buffer_load16<0>(r, dvo[j] - skip);
+      else lds_copy16(r, dst + (16 * w + RPI * j) * D, dvo[j] - skip);
+    };
+    auto land = [&](uint16_t* dst, const uint4* held) {
+      if constexpr (WIDEN) {
+#pragma unroll
+        for (int j = 0; j < NI; ++j) {
+          const int lr = RPI * j + lane / CPRD;
+          const int c = 2 * (lane % CPRD);  // the two 8-element chunks of this lane's 16 bytes
+          uint16_t* const row = dst + (16 * w + lr) * D;
+          *reinterpret_cast<uint4*>(row + 8 * (c ^ pf_swz<D>(lr))) =
+              KV::operand(raw_t{held[j].x, held[j].y});
+          *reinterpret_cast<uint4*>(row + 8 * ((c + 1) ^ pf_swz<D>(lr))) =
+              KV::operand(raw_t{held[j].z, held[j].w});
+        }
+      }
     };
     uint16_t* const k0 = &s_k0[grp][0];
     uint16_t* const k1 = &s_k1[grp][0];
@@ -909,9 +935,11 @@ __global__ __launch_bounds__(kPfThreads) void prefill_mfma_kernel(const PrefillP
       const TileCopy c = plan_tile(s_first, s_first < step_end);
 #pragma unroll
       for (int j = 0; j < NI; ++j) {
-        copy_rows(c.rk, c.skip, k0, j);
-        if (grp == 0) copy_rows(c.rv, c.skip, v0, j);  // group 1 copies V a step later
+        copy_rows(c.rk, c.skip, k0, k_held, j);
+        if (grp == 0) copy_rows(c.rv, c.skip, v0, v_held, j);  // group 1 copies V a step later
       }
+      land(k0, k_held);
+      if (grp == 0) land(v0, v_held);
       // group 0 copies step i + 1 in iteration i; group 1, K of step i + 1 and V of step i
       ck = plan_tile(s_first + 2, s_first + 2 < step_end);
       cv = grp == 0 ? ck : c;
@@ -938,14 +966,16 @@ __global__ __launch_bounds__(kPfThreads) void prefill_mfma_kernel(const PrefillP
         r0(k_cur, step, full, [&] { cn = plan_tile(step + 4, step + 4 < step_end); });
         r1(k_cur, step, full, [&] {
 #pragma unroll
-          for (int j = 0; j < NI; ++j) copy_rows(ck.rk, ck.skip, k_nxt, j);
+          for (int j = 0; j < NI; ++j) copy_rows(ck.rk, ck.skip, k_nxt, k_held, j);
         });
         r2(v_cur, [&] {
 #pragma unroll
-          for (int j = 0; j < NI; ++j) copy_rows(ck.rv, ck.skip, v_nxt, j);
+          for (int j = 0; j < NI; ++j) copy_rows(ck.rv, ck.skip, v_nxt, v_held, j);
         });
         r3(v_cur);
         ck = cn;
+        land(k_nxt, k_held);
+        land(v_nxt, v_held);
       }
       __builtin_amdgcn_s_waitcnt(kWaitVm0);
       __syncthreads();  // this iteration's copies landed; the reads of their slots are done
@@ -962,12 +992,12 @@ __global__ __launch_bounds__(kPfThreads) void prefill_mfma_kernel(const PrefillP
       if (i > 0 && step - 2 < step_end) {  // the second half of step i - 1
         r2(v_prv, [&] {
 #pragma unroll
-          for (int j = 0; j < NI; ++j) copy_rows(ck.rk, ck.skip, k_nxt, j);
+          for (int j = 0; j < NI; ++j) copy_rows(ck.rk, ck.skip, k_nxt, k_held, j);
         });
         r3(v_prv);
       } else {
 #pragma unroll
-        for (int j = 0; j < NI; ++j) copy_rows(ck.rk, ck.skip, k_nxt, j);
+        for (int j = 0; j < NI; ++j) copy_rows(ck.rk, ck.skip, k_nxt, k_held, j);
       }
       if (step < step_end) {
         const bool full = step_full(step);
@@ -978,11 +1008,13 @@ __global__ __launch_bounds__(kPfThreads) void prefill_mfma_kernel(const PrefillP
         });
         r1(k_cur, step, full, [&] {
 #pragma unroll
-          for (int j = 0; j < NI; ++j) copy_rows(cv.rv, cv.skip, v_cur, j);
+          for (int j = 0; j < NI; ++j) copy_rows(cv.rv, cv.skip, v_cur, v_held, j);
         });
         ck = ckn;
         cv = cvn;
+        land(v_cur, v_held);
       }
+      land(k_nxt, k_held);
       __builtin_amdgcn_s_waitcnt(kWaitVm0);
       __syncthreads();  // this iteration's copies landed; the reads of their slots are done
     };
@@ -1293,15 +1325,33 @@ __global__ __launch_bounds__(kPfFoldThreads) void prefill_sk_fold_kernel(const P
       make_uint2(Pack2<T>::pack(a.x * inv, a.y * inv), Pack2<T>::pack(a.z * inv, a.w * inv));
 }
 
+// Whether tasks over an fp8 cache are staged step by step: at most 768 keys a task (six key-step
+// pairs), where the schedule's half step after the last costs more than it hides. Measured
+// both ways: 300 queries over 300 keys (4 x H28/KVH4/D128) 22.2 against 23.7 us, 700 over a
+// 512-key window (H32/KVH8/D128) 41.2 against 42.9; 100 over 3000 keys 40.6 against 38.3, 700
+// over 4000 (4 x H28/KVH4) 259 against 223.
+inline bool pf_stepwise(const PrefillParams& p) {
+  const int seen = p.window > 0 ? p.window + kPfRows / p.G + 1 : p.max_ctx;
+  return (seen < p.max_ctx ? seen : p.max_ctx) <= 768;
+}
+
 template <typename T, typename KT>
 hipError_t launch_prefill_mfma_impl(const PrefillParams& p, int D, hipStream_t stream,
                                     bool* supported) {
   *supported = D == 64 || D == 128;
   if (!*supported) return hipSuccess;
   const dim3 grid(static_cast<unsigned>(p.sk_groups > 0 ? p.sk_groups : kXcds * p.xcd_per));
-  if (D == 128)
+  constexpr bool kFp8 = std::is_same<KT, fp8_t>::value;
+  const bool stepwise = kFp8 && pf_stepwise(p);
+  if (D == 128 && stepwise)
+    hipLaunchKernelGGL((prefill_mfma_kernel<T, KT, 128, kPfRB, false, kFp8>), grid, dim3(kPfThreads),
+                       0, stream, p);
+  else if (D == 128)
     hipLaunchKernelGGL((prefill_mfma_kernel<T, KT, 128, kPfRB, false>), grid, dim3(kPfThreads), 0,
                        stream, p);
+  else if (stepwise)
+    hipLaunchKernelGGL((prefill_mfma_kernel<T, KT, 64, kPfRB, false, kFp8>), grid, dim3(kPfThreads),
+                       0, stream, p);
   else
     hipLaunchKernelGGL((prefill_mfma_kernel<T, KT, 64, kPfRB, false>), grid, dim3(kPfThreads), 0,
                        stream, p);
@@ -1326,11 +1376,12 @@ hipError_t launch_prefix_partials_impl(const PrefillParams& p, int D, hipStream_
   *supported = D == 64 || D == 128;
   if (!*supported) return hipSuccess;
   const dim3 grid(static_cast<unsigned>(p.rblocks * p.KVH), static_cast<unsigned>(p.npart), 1);
+  constexpr bool kFp8 = std::is_same<KT, fp8_t>::value;  // key partitions are of few steps
   if (D == 128)
-    hipLaunchKernelGGL((prefill_mfma_kernel<T, KT, 128, kPfRB, true>), grid, dim3(kPfThreads), 0,
+    hipLaunchKernelGGL((prefill_mfma_kernel<T, KT, 128, kPfRB, true, kFp8>), grid, dim3(kPfThreads), 0,
                        stream, p);
   else
-    hipLaunchKernelGGL((prefill_mfma_kernel<T, KT, 64, kPfRB, true>), grid, dim3(kPfThreads), 0,
+    hipLaunchKernelGGL((prefill_mfma_kernel<T, KT, 64, kPfRB, true, kFp8>), grid, dim3(kPfThreads), 0,
                        stream, p);
   return hipGetLastError();
 }
