@@ -533,10 +533,18 @@ struct PartialsPlan {
   int kind;
 };
 
+// Whether a sliding window's size, not the table's, sets a decode's route and partitions. Not
+// over an fp8 cache at 4 rows per tile and head_dim 128, whose widening work wants the long
+// runs of stream-K and of the wide shape: 64 x H32/KVH8 under a 1024-token window 33.5 us
+// against 34.8 (wide partitions of the window) and 36.0 (regular ones).
+bool windows_shrink(bool kv_fp8, int RT, int head_dim, int window) {
+  return window > 0 && !(kv_fp8 && RT == 4 && head_dim == 128);
+}
+
 PartialsPlan plan_partials(const void* query, int q_dtype, int kv_dtype, int head_dim,
                            int block_size, int64_t slot_stride, bool rows16, int batch,
                            int q_len, int num_heads, int num_kv_heads, int max_context,
-                           bool has_out, int key_lo) {
+                           bool has_out, int key_lo, int window) {
   PartialsPlan pl;
   const int rows = q_len * (num_heads / num_kv_heads);
   pl.use_mfma = mfma_decode_route_ok(query, q_dtype, kv_dtype, head_dim, block_size, slot_stride,
@@ -545,20 +553,28 @@ PartialsPlan plan_partials(const void* query, int q_dtype, int kv_dtype, int hea
   // Decode with enough work to fill the chip: stream-K over every (sequence, KV head)
   // tile run, one workgroup per CU. Small decodes keep the partition kernel, whose short
   // runs start faster.
-  const int64_t tile_capacity =
-      static_cast<int64_t>(batch) * num_kv_heads * ceil_div(max_context, 16);
+  const int64_t triples = static_cast<int64_t>(batch) * num_kv_heads * ceil_div(rows, pl.RT);
+  const bool merges = has_out && key_lo == 0 && kFusedMerge && triples <= kMaxTickets;
+  // A sliding window counts for what it shows: 32 sequences of 16k tokens under a 1024-token
+  // window (H32/KVH8/D128 fp16) take 30.9 us on stream-K and the merge, 27.7 on the partition
+  // kernel; 64 under a 128-token one 22.1 and 17.6.
+  const bool windowed = merges && windows_shrink(kv_dtype == MSATTN_FP8_E4M3, pl.RT, head_dim, window) &&
+                        window < max_context;
+  const int seen = windowed ? window : max_context;
+  const int64_t tile_capacity = static_cast<int64_t>(batch) * num_kv_heads * ceil_div(seen, 16);
   const bool kv_fp8 = kv_dtype == MSATTN_FP8_E4M3;
+  // (under a window the fp8 cache at 8 rows per tile crosses earlier: 64 x H14/KVH2/D64 and a
+  // 4096-token window 30.6 us on stream-K, 32.6 on the partition kernel)
   const int64_t sk_min_tiles =
-      kv_fp8 && q_dtype != MSATTN_F32 && pl.RT == 8 ? kStreamKMinTilesFp8Rt8
+      kv_fp8 && q_dtype != MSATTN_F32 && pl.RT == 8 ? kStreamKMinTilesFp8Rt8 / (windowed ? 2 : 1)
       : head_dim == 64                               ? kStreamKMinTilesD64
                                                      : kStreamKMinTiles;
-  const int64_t triples = static_cast<int64_t>(batch) * num_kv_heads * ceil_div(rows, pl.RT);
   if (pl.use_mfma && q_len == 1 && batch <= kSkMaxBatch && tile_capacity >= sk_min_tiles)
     pl.kind = 1;
   // With an output to write, the MFMA partition kernel merges in-kernel (the last
   // partition of each (sequence, KV head, row tile) to finish folds the others in), so
   // no merge launch follows; it needs one header ticket per such triple.
-  else if (pl.use_mfma && has_out && key_lo == 0 && kFusedMerge && triples <= kMaxTickets)
+  else if (pl.use_mfma && merges)
     pl.kind = 2;
   else
     pl.kind = 0;
@@ -597,7 +613,7 @@ int partials_impl(const void* query, const void* k_cache, const void* v_cache,
   const PartialsPlan plan =
       plan_partials(query, q_dtype, kv_dtype, head_dim, block_size, cache_slot_stride, rows16,
                     batch, q_len, num_heads, num_kv_heads, max_context, fused_out != nullptr,
-                    key_lo);
+                    key_lo, window);
   const bool use_mfma = plan.use_mfma;
   const int RT = plan.RT;
   char* ws = static_cast<char*>(workspace);
@@ -632,6 +648,7 @@ int partials_impl(const void* query, const void* k_cache, const void* v_cache,
   p.sk_group = 1;
   p.sk_unit_groups = 0;
   p.sk_min_chunk = kSkMinChunk;
+  p.win_first = 0;
   p.mfma_waves = kMfmaWaves;
   p.mfma_deep = 0;
   p.key_lo = key_lo;
@@ -701,7 +718,8 @@ int partials_impl(const void* query, const void* k_cache, const void* v_cache,
     // 22.4 -> 20.7, 8 x H32/KVH8 at 3500 27.3 -> 24.9, level at 3936 and 5 x 5100. Shorter
     // wide partitions, and wide workgroups two to a CU, measured slower than the regular shape.
     if (kWideRoute && q_len == 1 && (RT == 4 || RT == 8) && q_dtype != MSATTN_F32 &&
-        kv_dtype != MSATTN_F32) {
+        kv_dtype != MSATTN_F32 &&
+        (!windows_shrink(kv_fp8, RT, head_dim, p.window) || p.window >= kPartWide)) {
       const int64_t triples = static_cast<int64_t>(batch) * num_kv_heads * p.rtiles;
       const int64_t want = static_cast<int64_t>(device_cus()) * kWideSlotsPct / 100;
       const int64_t np = std::max<int64_t>(1, want / triples);
@@ -716,6 +734,25 @@ int partials_impl(const void* query, const void* k_cache, const void* v_cache,
         p.part = kPartWide;
         p.max_parts = ceil_div(max_context, kPartWide);
         p.mfma_waves = kWideWaves;
+      }
+    }
+    // Under a window: the tiles it can touch in equal partitions from its first tile on, as
+    // long as the size the launch would take for a context of that length (never more slots a
+    // row than the workspace holds). The empty partitions below the window were launched,
+    // stored and merged before: 8 x H28/KVH4/D128, 4 queries over 16k tokens under a 1024-token
+    // window 39.4 -> 21.8 us, one query 23.3 -> 18.3.
+    const int64_t shown = static_cast<int64_t>(p.window) + q_len - 1;
+    if (windows_shrink(kv_fp8, RT, head_dim, p.window) && shown < max_context) {
+      const int tiles = ceil_div(static_cast<int>(shown) + 15, 16);
+      int most = p.part;
+      if (p.mfma_waves == kMfmaWaves && p.part == L.part)
+        most = choose_partition(batch, q_len, num_heads, num_kv_heads, static_cast<int>(shown));
+      const int n = ceil_div(16 * tiles, most);
+      const int part_tiles = ceil_div(ceil_div(tiles, n), p.mfma_waves) * p.mfma_waves;
+      if (ceil_div(tiles, part_tiles) <= p.max_parts) {
+        p.part = 16 * part_tiles;
+        p.max_parts = ceil_div(tiles, part_tiles);
+        p.win_first = 1;
       }
     }
   }
@@ -980,7 +1017,7 @@ int choose_route(const void* query, const void* out, const void* k_cache, const 
     return MSATTN_ROUTE_PREFILL_ANY;
   const PartialsPlan pl =
       plan_partials(query, q_dtype, kv_dtype, head_dim, block_size, cache_slot_stride, rows16,
-                    batch, q_len, num_heads, num_kv_heads, max_context, true, 0);
+                    batch, q_len, num_heads, num_kv_heads, max_context, true, 0, 0);
   if (pl.kind == 1) return MSATTN_ROUTE_STREAMK;
   if (pl.kind == 2) return MSATTN_ROUTE_PARTITION_FUSED;
   return pl.use_mfma ? MSATTN_ROUTE_PARTITION : MSATTN_ROUTE_GENERIC;

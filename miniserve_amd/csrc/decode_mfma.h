@@ -716,19 +716,22 @@ __global__ __launch_bounds__(W * kWave) void decode_mfma_kernel(const SplitParam
     b = blockIdx.z;
   }
 
+  int ctx = p.lens[b];
+  ctx = ctx < 0 ? 0 : (ctx > p.max_ctx ? p.max_ctx : ctx);
+  // Under a window the partitions begin at the window's first tile: the launch holds what the
+  // window shows in equal parts instead of the whole table (SplitParams::win_first).
+  const int tile0 = p.win_first ? max(0, ctx - p.q_len - p.window + 1) / 16 : 0;
   // Wave w owns a fixed run of the partition's tiles, so their page ids can be
-  // requested together with the context length instead of after it.
+  // requested together with the context length instead of after it (without a window).
   const int per_wave = p.part / (16 * kWaves);
-  const int tw0 = part * (p.part / 16) + w * per_wave;
+  const int tw0 = tile0 + part * (p.part / 16) + w * per_wave;
   int phys_pre = -1;
   if (lane < per_wave) {
     const int pg = ((tw0 + lane) * 16) / p.bs;
     if (pg < p.W) phys_pre = p.table[static_cast<int64_t>(b) * p.W + pg];
   }
 
-  int ctx = p.lens[b];
-  ctx = ctx < 0 ? 0 : (ctx > p.max_ctx ? p.max_ctx : ctx);
-  const int nparts = ctx > 0 ? ceil_div(ctx, p.part) : 1;
+  const int nparts = ctx > 0 ? ceil_div(ctx - 16 * tile0, p.part) : 1;
   if (part >= nparts) return;
 
   const int row0 = rtile * RT;
@@ -739,7 +742,7 @@ __global__ __launch_bounds__(W * kWave) void decode_mfma_kernel(const SplitParam
   const int i_last = (row0 + nrows - 1) / p.G;
   const int lo_all = max(p.key_lo, p.window > 0 ? max(0, ctx - p.q_len + i_first - p.window + 1) : 0);
   const int hi_all = p.causal ? min(ctx, ctx - p.q_len + i_last + 1) : ctx;
-  const int tok0 = part * p.part;
+  const int tok0 = 16 * tile0 + part * p.part;
   const int a0 = max(tok0, lo_all);
   const int a1 = min(min(tok0 + p.part, ctx), hi_all);
 

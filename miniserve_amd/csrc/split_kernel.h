@@ -107,6 +107,9 @@ struct SplitParams {
   // its partials and write the output; `tickets` are the header's arrival counters.
   void* out;
   int* tickets;
+  // In-kernel merge under a sliding window: a sequence's max_parts partitions begin at the
+  // tile of its window's first key (0: at its first token).
+  int win_first;
   int mfma_waves;  // partition MFMA kernel: waves per workgroup (4, or 8 for long partitions)
   int mfma_deep;   // partition MFMA kernel, regular shape at head_dim 64: the deeper residency
   int head_dim;    // the row's head size (the generic kernel's element mode compiles a larger
