@@ -108,9 +108,13 @@ size_t msattn_workspace_bytes(int batch, int q_len, int num_heads, int num_kv_he
  * (q_len 1, or at most 16 query rows per KV head) runs on the MFMA kernels for a bf16/fp16
  * query over a cache of its type, fp8 e4m3 or fp32, and for an fp32 query over any cache
  * (head_dim 64 or 128, 16-byte aligned query, cache pointers and strides on 16-byte
- * boundaries, block_size a multiple of 16); an fp32 query's chunked prefill (more than 16
- * query rows per KV head) also runs there. Other pairs and shapes take the generic kernel,
- * which needs only element-aligned caches. msattn_paged_attention_route names the route.
+ * boundaries, block_size a multiple of 16). A chunk of more than 16 query rows per KV head
+ * that the prefill kernel below does not take (an fp32 query, other head sizes, type pairs,
+ * page sizes and alignments) runs on the any-layout prefill kernel where a cost model in
+ * sizes prefers it, writing the output directly (or through a fold launch), else on the
+ * partition kernel (an fp32 query) or the generic kernel, which needs only element-aligned
+ * caches. msattn_paged_attention_route names the route; it has no window argument, and a
+ * windowed decode is routed by what its window shows, not by its table.
  * Runs msattn_paged_attention_partials followed by msattn_merge_partials, except:
  * chunked prefill on the MFMA kernel (bf16/fp16 query 16-byte aligned, output 8-byte
  * aligned, cache of the query's type, fp8 e4m3 or fp32, head_dim 64 or 128, more than 16

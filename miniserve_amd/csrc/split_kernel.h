@@ -50,7 +50,8 @@ constexpr int kPartMax = MSATTN_PART_MAX;
 // partials kernel used, so the merge can read it back.
 //   hdr[0] kind: 0 = per-row slots closed by end markers (partition kernels);
 //                1 = stream-K pieces (decode_streamk.h);
-//                2 = partition kernel that merged in-kernel and wrote the output
+//                2 = the launch wrote the output: the partition kernel merging in-kernel, or
+//                    the any-layout prefill kernel
 //   kind 1 also: hdr[1] sumT, [2] chunk c, [3] sub-ranges, [4] UG, [5] NUG, [6] B,
 //   [7] RT, and hdr[kHdrPrefix + b] = tiles of sequences before b (b = 0..B).
 //   A chunked prefill on the prefill kernel's stream-K schedule writes hdr[kHdrPrefix + t]
