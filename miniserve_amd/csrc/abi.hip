@@ -581,6 +581,13 @@ PartialsPlan plan_partials(const void* query, int q_dtype, int kv_dtype, int hea
   return pl;
 }
 
+// Whether the kernel a plan takes is built with the fused append: the partition and stream-K
+// kernels for a bf16/fp16 query at up to 8 query rows per tile, stream-K not over an fp8 cache.
+bool append_built(const PartialsPlan& plan, int q_dtype, int kv_dtype) {
+  return (q_dtype == MSATTN_BF16 || q_dtype == MSATTN_F16) && plan.RT <= 8 &&
+         (plan.kind == 2 || (plan.kind == 1 && kv_dtype != MSATTN_FP8_E4M3));
+}
+
 int partials_impl(const void* query, const void* k_cache, const void* v_cache,
                   int64_t cache_block_stride, int64_t cache_slot_stride,
                   int64_t cache_head_stride, const int32_t* block_table,
@@ -614,6 +621,8 @@ int partials_impl(const void* query, const void* k_cache, const void* v_cache,
       plan_partials(query, q_dtype, kv_dtype, head_dim, block_size, cache_slot_stride, rows16,
                     batch, q_len, num_heads, num_kv_heads, max_context, fused_out != nullptr,
                     key_lo, window);
+  // (a kernel without the append would leave the new token out of the cache and the output)
+  if (k_new != nullptr && !append_built(plan, q_dtype, kv_dtype)) return MSATTN_ERR_UNSUPPORTED;
   const bool use_mfma = plan.use_mfma;
   const int RT = plan.RT;
   char* ws = static_cast<char*>(workspace);
@@ -671,10 +680,8 @@ int partials_impl(const void* query, const void* k_cache, const void* v_cache,
   const hipStream_t st = static_cast<hipStream_t>(stream);
   if (plan.kind == 1) {  // stream-K
     *kind = 1;
-    if (k_new != nullptr) {  // fused append: the caller checked the route and types
-      p.k_new = k_new;
-      p.v_new = v_new;
-    }
+    p.k_new = k_new;  // fused append
+    p.v_new = v_new;
     const int units = num_kv_heads * p.rtiles;
     p.sk_group = largest_pow2_divisor_upto(
         units, sk_waves(kv_fp8 ? 1 : 2, q_dtype == MSATTN_F32 ? 4 : 2));
@@ -691,10 +698,8 @@ int partials_impl(const void* query, const void* k_cache, const void* v_cache,
     *kind = 2;
     p.out = fused_out;
     p.tickets = p.hdr + kHdrTickets;
-    if (k_new != nullptr) {  // fused append: the caller checked append_fusable
-      p.k_new = k_new;
-      p.v_new = v_new;
-    }
+    p.k_new = k_new;  // fused append
+    p.v_new = v_new;
     // The fp32 16-row route (P.V on the matrix core; its kernel unrolls kPartLongF32
     // tokens per workgroup) takes partitions of up to kPartLongF32 tokens when the grid
     // still reaches kTargetSlots: chunked prefill. Only the in-kernel merge reads these
@@ -1471,17 +1476,15 @@ int msattn_paged_attention_append(const void* query, const void* k_new, const vo
     return MSATTN_ERR_INVALID_ARG;
   if (!geometry_ok(batch, 1, num_heads, num_kv_heads, head_dim, max_context))
     return MSATTN_ERR_INVALID_ARG;
-  const int route = choose_route(query, out, k_cache, v_cache, cache_block_stride,
-                                 cache_slot_stride, cache_head_stride, batch, 1, num_heads,
-                                 num_kv_heads, head_dim, block_size, max_context, q_dtype,
-                                 kv_dtype, workspace_bytes);
-  // The partition and stream-K kernels built with the append: a bf16/fp16 query at up to
-  // 8 query rows per KV head (stream-K: not over an fp8 cache).
-  const bool append_kernel = (q_dtype == MSATTN_BF16 || q_dtype == MSATTN_F16) &&
-                             mfma_rows_per_tile(num_heads / num_kv_heads) <= 8;
-  if (kFusedAppend && append_kernel && aligned(k_new, 16) && aligned(v_new, 16) &&
-      (route == MSATTN_ROUTE_PARTITION_FUSED ||
-       (route == MSATTN_ROUTE_STREAMK && kv_dtype != MSATTN_FP8_E4M3))) {
+  // The plan the decode below runs by, window included: the append is fused only where that
+  // plan's kernel is built with it.
+  const PartialsPlan plan = plan_partials(
+      query, q_dtype, kv_dtype, head_dim, block_size, cache_slot_stride,
+      cache_rows16(k_cache, v_cache, cache_block_stride, cache_slot_stride, cache_head_stride,
+                   head_dim, kv_dtype),
+      batch, 1, num_heads, num_kv_heads, max_context, true, 0, window);
+  if (kFusedAppend && append_built(plan, q_dtype, kv_dtype) && aligned(k_new, 16) &&
+      aligned(v_new, 16)) {
     return attention_impl(query, k_cache, v_cache, cache_block_stride, cache_slot_stride,
                           cache_head_stride, block_table, context_lens, out, workspace,
                           workspace_bytes, batch, 1, num_heads, num_kv_heads, head_dim,

@@ -66,9 +66,23 @@ CASES = {
                                        "stream-K"),
     "stream-K table, fp16 D64 G7 window": (14, 2, 64, torch.float16, torch.float16, 64, 1024,
                                            1000, "stream-K"),
+    # a window that shows enough tiles for stream-K, whose kernel has no append over fp8, over a
+    # table below that line without the window (two launches)
+    "fp8 G7 D128, window at the stream-K line": (28, 4, 128, torch.bfloat16, torch.float8_e4m3fn,
+                                                 32, 384, 4096, "partition-fused"),
+    "fp8 G7 D64, window at the stream-K line": (14, 2, 64, torch.bfloat16, torch.float8_e4m3fn,
+                                                64, 384, 4096, "partition-fused"),
+    # a window that shows a stream-K launch over a 16-bit cache: the append in that launch
+    "bf16 window, stream-K": (32, 8, 128, torch.bfloat16, torch.bfloat16, 64, 160, 2100,
+                              "stream-K"),
     "head_dim 80, generic kernel (two launches)": (8, 2, 80, torch.bfloat16, torch.bfloat16, 8,
                                                    64, 0, "generic"),
 }
+
+
+# The kind word of the workspace header after the call (1 stream-K, 2 the partition kernel).
+KIND = {"fp8 G7 D128, window at the stream-K line": 1, "fp8 G7 D64, window at the stream-K line": 1,
+        "bf16 window, stream-K": 1}
 
 
 @pytest.mark.parametrize("name", list(CASES))
@@ -103,6 +117,7 @@ def test_append_equals_write_kv_then_decode(device, name):
         out = paged_attention_append(q, kn, vn, kc_a, vc_a, td, ld, max_context=cap,
                                      window=window or None, workspace=ws)
         torch.cuda.synchronize()
+        assert KIND.get(name, int(ws[:4].view(torch.int32))) == int(ws[:4].view(torch.int32))
         assert torch.equal(kc_a.view(torch.uint8), kc_b.view(torch.uint8)), "K caches differ"
         assert torch.equal(vc_a.view(torch.uint8), vc_b.view(torch.uint8)), "V caches differ"
         assert not torch.isnan(out.float()).any()
@@ -146,4 +161,36 @@ def test_runner_fused_append_equals_two_calls(device):
         assert torch.equal(a, b), f"step {step}"
         for x, y in zip(lf, lp):
             assert torch.equal(x.k_cache, y.k_cache) and torch.equal(x.v_cache, y.v_cache)
+        ctx = [c + 1 for c in ctx]
+
+
+def test_runner_fused_append_fp8_under_a_window(device):
+    """The graphed runner over an fp8 cache, a window at the stream-K line over a table below
+    it: the same outputs and caches with the fused call and with two calls."""
+    H, KVH, D, B, WIDTH = 14, 2, 64, 64, 384
+
+    def build(fused):
+        g = torch.Generator(device).manual_seed(5)
+        pa = PagedAttention(H, KVH, D, num_blocks=B * WIDTH, block_size=16, dtype=torch.bfloat16,
+                            kv_dtype=torch.float8_e4m3fn, device=device, window=4096)
+        kc, vc = (torch.randn(B * WIDTH, 16, KVH, D, generator=g, device=device)
+                  .to(torch.float8_e4m3fn) for _ in range(2))
+        layer = DecodeLayer(pa, kc, vc)
+        return GraphedDecodeRunner([layer], table_width=WIDTH, buckets=(B,),
+                                   fused_append=fused), layer
+
+    (fused, lf), (plain, lp) = build(True), build(False)
+    g = torch.Generator().manual_seed(6)
+    pages = torch.randperm(B * WIDTH, generator=g).view(B, WIDTH)
+    ctx = [int(x) for x in torch.randint(1, 16 * WIDTH - 8, (B,), generator=g)]
+    for step in range(3):
+        note(f"runner fp8 window step {step}: ctx={ctx[:6]}")
+        q, k, v = (torch.randn(1, B, 1, h, D, generator=g).to(torch.bfloat16).to(device)
+                   for h in (H, KVH, KVH))
+        a = fused.decode(q, k, v, pages.tolist(), ctx)
+        b = plain.decode(q, k, v, pages.tolist(), ctx)
+        torch.cuda.synchronize()
+        assert torch.equal(a, b), f"step {step}"
+        for x, y in ((lf.k_cache, lp.k_cache), (lf.v_cache, lp.v_cache)):
+            assert torch.equal(x.view(torch.uint8), y.view(torch.uint8))
         ctx = [c + 1 for c in ctx]
