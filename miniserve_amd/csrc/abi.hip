@@ -715,13 +715,22 @@ int partials_impl(const void* query, const void* k_cache, const void* v_cache,
       }
     }
     // Few (sequence, KV head, row tile) triples over long contexts: when kPartWide-token
-    // partitions give about a workgroup per CU or more (the last of them possibly short), and
-    // the launch stays within 1.5 workgroups per CU, the partition kernel's wide shape (8
-    // waves, two per SIMD). Its two waves per SIMD fill each other's waits (C5-decode: 24.1 ->
-    // 22.6 us). A table that ends inside the last partition counts: 16 x H28/KVH4/D128 at 3500
-    // tokens 30.0 -> 25.9 us (fp8 cache 26.0 -> 21.1), 12 x 5100 31.8 -> 27.3, 24 x 1040
-    // 22.4 -> 20.7, 8 x H32/KVH8 at 3500 27.3 -> 24.9, level at 3936 and 5 x 5100. Shorter
-    // wide partitions, and wide workgroups two to a CU, measured slower than the regular shape.
+    // partitions give about a workgroup per CU or more, and the launch stays within 1.5
+    // workgroups per CU, the partition kernel's wide shape (8 waves, two per SIMD). Its two
+    // waves per SIMD fill each other's waits (C5-decode: 24.1 -> 22.6 us). Shorter wide
+    // partitions, and wide workgroups two to a CU, measured slower than the regular shape.
+    //
+    // A table that ends inside the np-th partition leaves waves of the last workgroups without
+    // tiles (wave w owns tiles 8 w .. 8 w + 7), which costs the less the fewer they are of all.
+    // Timed both ways on H32/KVH8 and H28/KVH4 at 128 dims and H14/KVH2 at 64, bf16 and fp8
+    // caches, contexts of 5/8 of the table up and full ones:
+    //   np >= 3: level to 36 % faster (16 x H28/KVH4 at 3584 tokens 29.2 -> 25.3 us);
+    //   np == 2: from 7/8 of both partitions, -20 to +4 %; at 1040 tokens up to 34 % slower;
+    //   np == 1 (one workgroup a triple, no merge): from half the partition where the launch
+    //     fills 80 to 100 % of the CUs, 2-32 % faster (32 x H32/KVH8 at 512 tokens 17.4 ->
+    //     15.0); with fewer or more triples, or a shorter table, up to 60 % slower in places
+    //     (288 x H28/KVH4 pairs at 320 tokens 13.7 -> 21.9 over fp8, 48 x H32/KVH8 at 128
+    //     tokens 14.2 -> 16.5).
     if (kWideRoute && q_len == 1 && (RT == 4 || RT == 8) && q_dtype != MSATTN_F32 &&
         kv_dtype != MSATTN_F32 &&
         (!windows_shrink(kv_fp8, RT, head_dim, p.window) || p.window >= kPartWide)) {
@@ -734,7 +743,14 @@ int partials_impl(const void* query, const void* k_cache, const void* v_cache,
       // (5-10 % faster on H32/KVH8 decodes of 6-20 workgroups per CU); at 8 rows per tile,
       // at head_dim 64 and over a 16-bit cache the cap stands (7-18 % slower without it).
       const bool uncapped = kWideFp8Uncapped && kv_fp8 && RT == 4 && head_dim == 128;
-      if (ceil_div(max_context, kPartWide) >= np &&
+      // (uncapped launches past 1.5 workgroups per CU: 15-23 % faster from 9/16 of a partition)
+      const bool filled =
+          max_context >= np * kPartWide ||
+          (np >= 3   ? ceil_div(max_context, kPartWide) >= np
+           : np == 2 ? 8 * static_cast<int64_t>(max_context) >= 7 * np * kPartWide
+           : launched <= want ? 2 * max_context >= kPartWide && 10 * launched >= 8 * want
+                              : uncapped && 16 * max_context >= 9 * kPartWide && 2 * launched >= 3 * want);
+      if (filled &&
           (uncapped || 100 * launched <= static_cast<int64_t>(kWideMaxPct) * want)) {
         p.part = kPartWide;
         p.max_parts = ceil_div(max_context, kPartWide);
