@@ -757,17 +757,37 @@ int partials_impl(const void* query, const void* k_cache, const void* v_cache,
         p.mfma_waves = kWideWaves;
       }
     }
-    // Under a window: the tiles it can touch in equal partitions from its first tile on, as
-    // long as the size the launch would take for a context of that length (never more slots a
-    // row than the workspace holds). The empty partitions below the window were launched,
-    // stored and merged before: 8 x H28/KVH4/D128, 4 queries over 16k tokens under a 1024-token
-    // window 39.4 -> 21.8 us, one query 23.3 -> 18.3.
+    // Under a window: the tiles it can touch in equal partitions from its first tile on (never
+    // more slots a row than the workspace holds). The empty partitions below the window were
+    // launched, stored and merged before: 8 x H28/KVH4/D128, 4 queries over 16k tokens under a
+    // 1024-token window 39.4 -> 21.8 us, one query 23.3 -> 18.3. (The wide shape and the fp32
+    // route's long partitions are still taken by the table, above, and then cut to the window.)
+    //
+    // Their size, for the regular shape: the smallest whose launch stays within kTargetSlots
+    // workgroups (two a CU, one round). A window that begins inside a tile touches one tile more
+    // than its length holds, so that sizes that reach the target, as without a window, ran a few
+    // workgroups into a second round (4 x H14/KVH2/D64 under 4096 tokens, 520 workgroups: 21.1 us
+    // against 15.0 with 264). One partition a row, which writes the output without a merge:
+    // whatever fits one where the rows fill 80 % of the CUs (32 x 4 queries of H32/KVH8 under 128
+    // tokens 10.0 us against 15.5 in two), up to two tiles a wave where they fill half of them
+    // (25 x 4 fp32 queries of H28/KVH4 under 54 tokens 13.8 against 18.5). At most 16 of the
+    // smallest size, or at 16 rows a tile: the merge reads them all (4 x H28/KVH4 fp32 under 1590
+    // tokens 22.9 us in 26 of 64 tokens, 18.7 in 13 of 128).
     const int64_t shown = static_cast<int64_t>(p.window) + q_len - 1;
     if (windows_shrink(kv_fp8, RT, head_dim, p.window) && shown < max_context) {
       const int tiles = ceil_div(static_cast<int>(shown) + 15, 16);
+      const int64_t triples = static_cast<int64_t>(batch) * num_kv_heads * p.rtiles;
       int most = p.part;
-      if (p.mfma_waves == kMfmaWaves && p.part == L.part)
-        most = choose_partition(batch, q_len, num_heads, num_kv_heads, static_cast<int>(shown));
+      if (p.mfma_waves == kMfmaWaves && p.part == L.part) {
+        most = kPartMax;
+        const int64_t cus = device_cus();
+        const int one = 10 * triples >= 8 * cus ? kPartMax : 2 * triples >= cus ? kPartMax / 4 : 0;
+        for (int part : kPartitionChoices) {
+          const int parts = ceil_div(16 * tiles, part);
+          const bool many = part <= kPartMax / 8 || (part <= kPartMax / 4 && RT == 16);
+          if (16 * tiles > one && triples * parts <= kTargetSlots && !(many && parts > 16)) most = part;
+        }
+      }
       const int n = ceil_div(16 * tiles, most);
       const int part_tiles = ceil_div(ceil_div(tiles, n), p.mfma_waves) * p.mfma_waves;
       if (ceil_div(tiles, part_tiles) <= p.max_parts) {

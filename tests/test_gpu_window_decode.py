@@ -53,3 +53,40 @@ def test_windowed_decode(device, H, KVH, D, B, q_len, pages, q_dtype, kv_dtype, 
         assert not o[0].any()
         err = np.abs(o - ref).max()
         assert err < (1e-4 if q_dtype == torch.float32 else 2e-2 * np.abs(ref).max())
+
+
+@pytest.mark.parametrize("H,KVH,D,B,q_len,pages,q_dtype,window,part,waves", [
+    (14, 2, 64, 4, 1, 512, torch.bfloat16, 4096, 128, 4),   # 65 of 64 tokens: 520 workgroups
+    (32, 8, 128, 4, 1, 128, torch.bfloat16, 1024, 128, 4),  # 17 of 64: 544
+    (32, 8, 128, 2, 1, 128, torch.bfloat16, 1000, 64, 4),   # 16 of 64, one round
+    (28, 4, 128, 4, 1, 298, torch.float32, 1590, 128, 4),   # more than 16 of 64
+    (32, 8, 128, 2, 4, 350, torch.bfloat16, 2553, 256, 4),  # 16 rows a tile: of 128
+    (32, 8, 128, 32, 4, 512, torch.bfloat16, 128, 192, 4),  # every CU has a row: one partition
+    (32, 8, 128, 16, 1, 64, torch.bfloat16, 100, 128, 4),   # half the CUs, two tiles a wave: one
+    (32, 8, 128, 2, 1, 64, torch.bfloat16, 100, 64, 4),     # fewer rows: two
+])
+def test_partitions_of_a_window(device, H, KVH, D, B, q_len, pages, q_dtype, window, part, waves):
+    """The size of a windowed launch's partitions (256 CUs): one round of workgroups, no more
+    partitions than a merge should read, one where that fills the launch."""
+    if torch.cuda.get_device_properties(device).multi_processor_count != 256:
+        pytest.skip("the sizes are of a 256-CU device")
+    cap = 16 * pages
+    print(f"[case] H={H}/{KVH} D={D} B={B} q_len={q_len} window={window}", flush=True)
+    g = torch.Generator().manual_seed(window)
+    lens = [cap, 1, cap - 7][:B] + [int(x) for x in torch.randint(1, cap + 1, (max(0, B - 3),), generator=g)]
+    pool = 2 * pages
+    q = torch.randn(B, q_len, H, D, generator=g).to(q_dtype)
+    kc, vc = (torch.randn(pool, 16, KVH, D, generator=g).to(q_dtype) for _ in range(2))
+    table = torch.randint(0, pool, (B, pages), generator=g)
+    ws = torch.zeros(nat.lib().msattn_workspace_bytes(B, q_len, H, KVH, D, cap), dtype=torch.uint8,
+                     device=device)
+    out = paged_attention(q.to(device), kc.to(device), vc.to(device), table.to(device, torch.int32),
+                          torch.tensor(lens, dtype=torch.int32, device=device), window=window,
+                          workspace=ws)
+    hdr = ws[:4 * (64 + 4096)].view(torch.int32).cpu()
+    assert (int(hdr[0]), int(hdr[8]), int(hdr[9])) == (2, part, waves), hdr[:16].tolist()
+    assert not hdr[64:].any()
+    rows = list(range(min(B, 3)))
+    ref = dense.paged_attention_f64(q[rows], kc, vc, table[rows], lens[:len(rows)], window=window)
+    err = np.abs(out[rows].double().cpu().numpy() - ref).max()
+    assert err < (1e-4 if q_dtype == torch.float32 else 2e-2 * np.abs(ref).max())
