@@ -541,6 +541,24 @@ bool windows_shrink(bool kv_fp8, int RT, int head_dim, int window) {
   return window > 0 && !(kv_fp8 && RT == 4 && head_dim == 128);
 }
 
+// Eighths of the stream-K threshold (in tiles of the table) from which the tiles a window shows
+// take stream-K: the partition kernel launches no empty partitions under a window, but its
+// partitions are shorter there. Timed both ways at 16,384 to 125,000 window tiles over 4k to 8k
+// tables, partition kernel over stream-K just below and at each line:
+//   head_dim 128: 16-bit 0.92 and 1.05 (64 x H28/KVH4 at 40,960 tiles 1.05, at 60,000 1.20); an
+//     fp32 cache at 8 rows per tile 0.89 and 1.01-1.06, at up to 4 0.99 and 1.03; an fp32 query
+//     over a 16-bit cache at up to 4 rows 0.95 and 1.08, at 8 below 1 all the way;
+//   head_dim 64 (H14/KVH2): 16-bit 0.95 and 1.06, an fp32 cache 0.93 and 1.02-1.05, an fp32 query
+//     over a narrower one below 1 all the way;
+//   a 16-bit query over fp8 at 8 rows per tile 0.86-0.99 and 1.07.
+int window_eighths(int q_dtype, int kv_dtype, int head_dim, int RT) {
+  const bool few_rows = head_dim == 128 && RT <= 4;
+  if (kv_dtype == MSATTN_FP8_E4M3) return q_dtype != MSATTN_F32 && RT == 8 ? 4 : 8;
+  if (kv_dtype == MSATTN_F32) return few_rows ? 6 : 3;
+  if (q_dtype == MSATTN_F32) return few_rows ? 6 : 8;
+  return head_dim == 128 ? 5 : 6;
+}
+
 PartialsPlan plan_partials(const void* query, int q_dtype, int kv_dtype, int head_dim,
                            int block_size, int64_t slot_stride, bool rows16, int batch,
                            int q_len, int num_heads, int num_kv_heads, int max_context,
@@ -563,12 +581,10 @@ PartialsPlan plan_partials(const void* query, int q_dtype, int kv_dtype, int hea
   const int seen = windowed ? window : max_context;
   const int64_t tile_capacity = static_cast<int64_t>(batch) * num_kv_heads * ceil_div(seen, 16);
   const bool kv_fp8 = kv_dtype == MSATTN_FP8_E4M3;
-  // (under a window the fp8 cache at 8 rows per tile crosses earlier: 64 x H14/KVH2/D64 and a
-  // 4096-token window 30.6 us on stream-K, 32.6 on the partition kernel)
-  const int64_t sk_min_tiles =
-      kv_fp8 && q_dtype != MSATTN_F32 && pl.RT == 8 ? kStreamKMinTilesFp8Rt8 / (windowed ? 2 : 1)
-      : head_dim == 64                               ? kStreamKMinTilesD64
-                                                     : kStreamKMinTiles;
+  int64_t sk_min_tiles = kv_fp8 && q_dtype != MSATTN_F32 && pl.RT == 8 ? kStreamKMinTilesFp8Rt8
+                         : head_dim == 64                              ? kStreamKMinTilesD64
+                                                                       : kStreamKMinTiles;
+  if (windowed) sk_min_tiles = sk_min_tiles * window_eighths(q_dtype, kv_dtype, head_dim, pl.RT) / 8;
   if (pl.use_mfma && q_len == 1 && batch <= kSkMaxBatch && tile_capacity >= sk_min_tiles)
     pl.kind = 1;
   // With an output to write, the MFMA partition kernel merges in-kernel (the last

@@ -90,3 +90,35 @@ def test_partitions_of_a_window(device, H, KVH, D, B, q_len, pages, q_dtype, win
     ref = dense.paged_attention_f64(q[rows], kc, vc, table[rows], lens[:len(rows)], window=window)
     err = np.abs(out[rows].double().cpu().numpy() - ref).max()
     assert err < (1e-4 if q_dtype == torch.float32 else 2e-2 * np.abs(ref).max())
+
+
+@pytest.mark.parametrize("H,KVH,D,B,window,q_dtype,kv_dtype,kind", [
+    (32, 8, 128, 32, 2544, torch.bfloat16, torch.bfloat16, 2),   # 40,704 tiles
+    (32, 8, 128, 32, 2560, torch.bfloat16, torch.bfloat16, 1),   # 40,960
+    (28, 4, 128, 32, 3056, torch.float32, torch.float32, 2),     # 24,448
+    (28, 4, 128, 32, 3072, torch.float32, torch.float32, 1),
+    (32, 8, 128, 32, 3072, torch.float32, torch.bfloat16, 1),    # 49,152
+    (28, 4, 128, 64, 3072, torch.float32, torch.bfloat16, 2),
+    (14, 2, 64, 192, 4080, torch.bfloat16, torch.bfloat16, 2),   # 97,920
+    (14, 2, 64, 192, 4096, torch.bfloat16, torch.bfloat16, 1),
+])
+def test_window_tiles_that_take_stream_k(device, H, KVH, D, B, window, q_dtype, kv_dtype, kind):
+    """The kernel on both sides of the lines in tiles a window shows, over a table past them."""
+    pages, cap = 264, 16 * 264
+    print(f"[case] H={H}/{KVH} D={D} B={B} window={window} {q_dtype}/{kv_dtype}", flush=True)
+    g = torch.Generator(device).manual_seed(window)
+    lens = torch.randint(1, cap + 1, (B,), generator=torch.Generator().manual_seed(B)).to(torch.int32)
+    lens[0], lens[1], lens[2] = cap, 0, window + 1
+    q = torch.randn(B, 1, H, D, generator=g, device=device).to(q_dtype)
+    kc, vc = (torch.randn(pages, 16, KVH, D, generator=g, device=device).to(kv_dtype)
+              for _ in range(2))
+    table = torch.randint(0, pages, (B, pages), generator=torch.Generator().manual_seed(1))
+    ws = torch.zeros(nat.lib().msattn_workspace_bytes(B, 1, H, KVH, D, cap), dtype=torch.uint8,
+                     device=device)
+    out = paged_attention(q, kc, vc, table.to(device, torch.int32), lens.to(device), window=window,
+                          workspace=ws)
+    assert int(ws[:4].view(torch.int32)) == kind
+    ref = dense.paged_attention_f64(q[:3].cpu(), kc.cpu(), vc.cpu(), table[:3], lens[:3].tolist(),
+                                    window=window, kv_cast=True)
+    err = np.abs(out[:3].double().cpu().numpy() - ref).max()
+    assert err < (1e-4 if q_dtype == torch.float32 else 2e-2 * np.abs(ref).max())
