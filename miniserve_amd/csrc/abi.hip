@@ -993,7 +993,8 @@ PaPlan prefill_any_plan(int batch, int q_len, int num_heads, int num_kv_heads, i
   const int64_t cus = device_cus();
   const int64_t P = std::max<int64_t>(1, ceil_div(ceil_div(max_context, kPfStep), 2));
   plan.cost_ns = (tasks + cus - 1) / cus * P * unit + kOneFixed;
-  if (tasks > kPaSkMaxTasks) return plan;
+  // (the work list's offsets are 32-bit)
+  if (tasks > kPaSkMaxTasks || tasks * (P + kPfSkHead) >= (int64_t(1) << 30)) return plan;
   const Layout L = workspace_layout(batch, q_len, num_heads, num_kv_heads, head_dim, max_context);
   const size_t ml_at = round256(sizeof(int) * (kHdrPrefix + static_cast<size_t>(tasks) + 2));
   const size_t per_share = static_cast<size_t>(2) * kPfRows * (2 + DP) * sizeof(float);

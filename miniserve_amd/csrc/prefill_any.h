@@ -280,7 +280,7 @@ __global__ __launch_bounds__(pa_groups(DP) * kPfGroupThreads) void prefill_any_k
     const int gtid = tid - grp * GT;
     const int hh = lane >> 5;
     const int cc = lane & 31;
-    int it_lo = 0, it_hi = 1 << 24;
+    int it_lo = 0, it_hi = 1 << 24;  // (2^24 units hold 2^31 keys)
     bool full = true;
     unsigned task;
     if (sk) {
@@ -360,7 +360,7 @@ __global__ __launch_bounds__(pa_groups(DP) * kPfGroupThreads) void prefill_any_k
     const int step0 = t.step_first * (kPfStep / KS);
     const int first = step0 + SPU * it_lo;
     const int end = t.hi_all > t.lo_all
-                        ? min((t.hi_all + KS - 1) / KS, step0 + SPU * min(it_hi, 1 << 20))
+                        ? min(ceil_div(t.hi_all, KS), step0 + SPU * it_hi)
                         : first;
 
     const int n_it = end > first ? (end - first + NG - 1) / NG : 0;

@@ -124,3 +124,25 @@ def test_shares(device, H, KVH, D, q_len, lens, q_dtype):
     print(f"[case] shares H={H}/{KVH} D={D} q_len={q_len} {q_dtype}", flush=True)
     q, kc, vc, table = make(H, KVH, D, lens, q_len, q_dtype, q_dtype, 16, q_len)
     check(device, q, kc, vc, table, lens, D)
+
+
+@pytest.mark.parametrize("q_dtype,rows", [(F32, 120), (BF16, 120)])
+def test_keys_past_2_27(device, q_dtype, rows):
+    """A context of 2^27 + 4096 tokens whose table repeats one page, its last page apart: keys of
+    score 0 and value 1, and a last page whose 4096 keys outweigh them with value 2. Every task
+    reads to its end. The softmax in closed form: n keys of weight 1, 4096 of weight e^s."""
+    D, bs, n = 8, 4096, 1 << 27
+    print(f"[case] {n + bs} keys, {q_dtype}", flush=True)
+    kc = torch.zeros(2, bs, 1, D, dtype=q_dtype, device=device)
+    vc = torch.ones(2, bs, 1, D, dtype=q_dtype, device=device)
+    kc[1], vc[1] = 1.0, 2.0
+    table = torch.zeros(1, n // bs + 1, dtype=torch.int32, device=device)
+    table[0, -1] = 1
+    q = torch.full((1, rows, 1, D), 1.5, dtype=q_dtype, device=device)  # s = 12
+    assert kernel_route(q, kc, table) == ROUTE
+    lens = torch.tensor([n + bs], dtype=torch.int32, device=device)
+    out = paged_attention(q, kc, vc, table, lens, causal=False, scale=1.0)
+    w = 4096 * np.exp(12.0)
+    want = (n + 2 * w) / (n + w)
+    # (every share's sums of ones are whole numbers below 2^24, so exact in fp32)
+    assert float((out.double() - want).abs().max()) / want < BAR[q_dtype]
