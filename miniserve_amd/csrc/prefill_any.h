@@ -21,11 +21,14 @@
 // (741-926 us: a second copy of the loop's products spills); wave priority for either group
 // or for the scores, and K operands read a product group ahead (576-581 us).
 //
-// 16-bit types: v_mfma_f32_32x32x16. The weights are kept to 16 bits more than one operand
-// holds: P = hi + lo, two operands of the query type, so that P V is summed over products
-// as exact as fp32 weights give after the output's rounding (the generic kernel's weights
-// are fp32). 256 queries over 512 to 2304 keys (H24/KVH8/D96 bf16): 30 us against the generic
-// kernel's 182; 4 x 256 queries over 4096 keys (H32/KVH8/D256): 0.38 ms against 7.5.
+// 16-bit types: v_mfma_f32_32x32x16. The weights are kept in two operands of the query type,
+// P = hi + lo, so that P V is summed over products as exact as the result's rounding needs (the
+// generic kernel's weights are fp32): 16 significant bits in bf16, 2^-8 of the result's own
+// rounding; 22 in fp16, whose lo is scaled by 2^18 and summed on its own, so that a weight is
+// held to 2^-43 of the row's largest rather than to fp16's smallest step, 2^-24 (a row whose
+// largest weight meets a zero value is made of the small ones). 256 queries over 512 to 2304
+// keys (H24/KVH8/D96 bf16): 30 us against the generic kernel's 182; 4 x 256 queries over 4096
+// keys (H32/KVH8/D256): 0.38 ms against 7.5.
 //
 // Lane layout (both): lane (cc = l % 32, hh = l / 32) holds query row cc. Register v of a
 // 32-key score tile is key (v & 3) + 8 (v >> 2) + 4 hh; register v of output tile t is dim
@@ -248,6 +251,8 @@ __global__ __launch_bounds__(pa_groups(DP) * kPfGroupThreads) void prefill_any_k
   constexpr int ND = DP / 32;
   constexpr int JD = F32 ? DP / 8 : DP / 16;  // K operand chunks of a lane
   constexpr int WROWS = 32;
+  // fp16's rest of a weight, scaled: weights are at most 2^8 (kPfSumBound), a rest 2^-4.
+  constexpr float kLoScale = std::is_same<T, _Float16>::value ? 0x1p18f : 1.0f;
 
   constexpr int kKBytes = KS * RSK * static_cast<int>(sizeof(T));
   constexpr int kVBytes = KS * RSV * static_cast<int>(sizeof(T));
@@ -547,7 +552,7 @@ __global__ __launch_bounds__(pa_groups(DP) * kPfGroupThreads) void prefill_any_k
               hi[k] = Pack2<T>::pack(x, y);
               float a, c;
               pa_unpack2<T>(hi[k], a, c);
-              lo[k] = Pack2<T>::pack(x - a, y - c);
+              lo[k] = Pack2<T>::pack((x - a) * kLoScale, (y - c) * kLoScale);
             }
             ph[tl][c2] = make_uint4(hi[0], hi[1], hi[2], hi[3]);
             pl[tl][c2] = make_uint4(lo[0], lo[1], lo[2], lo[3]);
@@ -580,21 +585,41 @@ __global__ __launch_bounds__(pa_groups(DP) * kPfGroupThreads) void prefill_any_k
           for (int c = 0; c < NC; ++c) acc[i + c] += o[c];
         }
       } else {
+        auto v_operand = [&](int tl, int c2, int i) {
+          uint16_t* lo = reinterpret_cast<uint16_t*>(vb) +
+                         (32 * tl + 16 * c2 + 4 * hh + tr_tok) * RSV + 32 * i + tr_dim;
+          const uint2 x = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4*)lo));
+          const uint2 y = __builtin_bit_cast(
+              uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4*)(lo + 8 * RSV)));
+          return make_uint4(x.x, x.y, y.x, y.y);
+        };
+        if constexpr (kLoScale == 1.0f) {
 #pragma unroll
-        for (int tl = 0; tl < NT; ++tl)
+          for (int tl = 0; tl < NT; ++tl)
 #pragma unroll
-          for (int c2 = 0; c2 < 2; ++c2)
+            for (int c2 = 0; c2 < 2; ++c2)
 #pragma unroll
-            for (int i = 0; i < ND; ++i) {
-              uint16_t* lo = reinterpret_cast<uint16_t*>(vb) +
-                             (32 * tl + 16 * c2 + 4 * hh + tr_tok) * RSV + 32 * i + tr_dim;
-              const uint2 x = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4*)lo));
-              const uint2 y = __builtin_bit_cast(
-                  uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4*)(lo + 8 * RSV)));
-              const uint4 va = make_uint4(x.x, x.y, y.x, y.y);
-              acc[i] = Mfma32<T>::mac(va, ph[tl][c2], acc[i]);
-              acc[i] = Mfma32<T>::mac(va, pl[tl][c2], acc[i]);
-            }
+              for (int i = 0; i < ND; ++i) {
+                const uint4 va = v_operand(tl, c2, i);
+                acc[i] = Mfma32<T>::mac(va, ph[tl][c2], acc[i]);
+                acc[i] = Mfma32<T>::mac(va, pl[tl][c2], acc[i]);
+              }
+        } else {  // the rests' products on their own, unscaled into the sum
+#pragma unroll
+          for (int i = 0; i < ND; ++i) {
+            mf_f32x16 o = zero16();
+#pragma unroll
+            for (int tl = 0; tl < NT; ++tl)
+#pragma unroll
+              for (int c2 = 0; c2 < 2; ++c2) {
+                const uint4 va = v_operand(tl, c2, i);
+                acc[i] = Mfma32<T>::mac(va, ph[tl][c2], acc[i]);
+                o = Mfma32<T>::mac(va, pl[tl][c2], o);
+              }
+#pragma unroll
+            for (int v = 0; v < 16; ++v) acc[i][v] = fmaf(o[v], 1.0f / kLoScale, acc[i][v]);
+          }
+        }
       }
     };
 

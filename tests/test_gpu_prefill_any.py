@@ -146,3 +146,23 @@ def test_keys_past_2_27(device, q_dtype, rows):
     want = (n + 2 * w) / (n + w)
     # (every share's sums of ones are whole numbers below 2^24, so exact in fp32)
     assert float((out.double() - want).abs().max()) / want < BAR[q_dtype]
+
+
+@pytest.mark.parametrize("q_dtype", [F16, BF16])
+@pytest.mark.parametrize("D,gap", [(96, 12.0), (32, 16.0), (200, 20.0)])
+def test_weights_far_below_the_largest(device, q_dtype, D, gap):
+    """An attention sink: key 0 outweighs every other by e^gap and its value is zero, so the
+    output is made of weights down to 2^-29 of the largest. (Values of 2^13 keep it a normal
+    fp16 number, so that the bar's rounding holds.)"""
+    H, KVH, q_len, lens = 3, 1, 127, [300]
+    print(f"[case] sink D={D} {q_dtype} gap={gap}", flush=True)
+    q, kc, vc, table = make(H, KVH, D, lens, q_len, q_dtype, q_dtype, 16, D)
+    at = int(table[0, 0])
+    q[..., 0] = 4.0
+    kc[..., 0] = 0
+    kc[at, 0] = 0
+    kc[at, 0, :, 0] = gap / 4.0 * D ** 0.5
+    vc *= 2.0 ** 13
+    vc[at, 0] = 0
+    check(device, q, kc, vc, table, lens, D)
+    check(device, q, kc, vc, table, lens, D, causal=False)
