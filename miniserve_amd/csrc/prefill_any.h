@@ -23,10 +23,12 @@
 //
 // 16-bit types: v_mfma_f32_32x32x16. The weights are kept in two operands of the query type,
 // P = hi + lo, so that P V is summed over products as exact as the result's rounding needs (the
-// generic kernel's weights are fp32): 16 significant bits in bf16, 2^-8 of the result's own
-// rounding; 22 in fp16, whose lo is scaled by 2^18 and summed on its own, so that a weight is
+// generic kernel's weights are fp32): 15 to 16 significant bits in bf16, 2^-7 of the result's
+// own rounding; 21 or more in fp16, whose lo is scaled by 2^18 and summed on its own, so that a weight is
 // held to 2^-43 of the row's largest rather than to fp16's smallest step, 2^-24 (a row whose
-// largest weight meets a zero value is made of the small ones). 256 queries over 512 to 2304
+// largest weight meets a zero value is made of the small ones). hi is rounded down and lo gets
+// 2^-24 of the weight on top, so that neither is below 0 nor is lo 0 beside a weight: an infinite
+// value then gives an infinite result, not the NaN of inf - inf or inf * 0. 256 queries over 512 to 2304
 // keys (H24/KVH8/D96 bf16): 30 us against the generic kernel's 182; 4 x 256 queries over 4096
 // keys (H32/KVH8/D256): 0.38 ms against 7.5.
 //
@@ -133,6 +135,15 @@ __device__ __forceinline__ void pa_unpack2(uint32_t w, float& a, float& b) {
     a = static_cast<float>(h.x);
     b = static_cast<float>(h.y);
   }
+}
+
+// Two weights (at least 0) rounded towards zero to T.
+template <typename T>
+__device__ __forceinline__ uint32_t pa_pack2_down(float a, float b) {
+  if constexpr (std::is_same<T, bf16_t>::value)
+    return __builtin_amdgcn_perm(__float_as_uint(b), __float_as_uint(a), 0x07060302u);
+  else
+    return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(a, b));
 }
 
 // Four output elements at o (dims d .. d + 3 of a row of D), as one store where VEC.
@@ -251,7 +262,7 @@ __global__ __launch_bounds__(pa_groups(DP) * kPfGroupThreads) void prefill_any_k
   constexpr int ND = DP / 32;
   constexpr int JD = F32 ? DP / 8 : DP / 16;  // K operand chunks of a lane
   constexpr int WROWS = 32;
-  // fp16's rest of a weight, scaled: weights are at most 2^8 (kPfSumBound), a rest 2^-4.
+  // fp16's rest of a weight, scaled: weights are at most 2^8 (kPfSumBound), a rest 2^-3.
   constexpr float kLoScale = std::is_same<T, _Float16>::value ? 0x1p18f : 1.0f;
 
   constexpr int kKBytes = KS * RSK * static_cast<int>(sizeof(T));
@@ -549,10 +560,11 @@ __global__ __launch_bounds__(pa_groups(DP) * kPfGroupThreads) void prefill_any_k
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
               const float x = pr[tl][8 * c2 + 2 * k], y = pr[tl][8 * c2 + 2 * k + 1];
-              hi[k] = Pack2<T>::pack(x, y);
+              hi[k] = pa_pack2_down<T>(x, y);
               float a, c;
               pa_unpack2<T>(hi[k], a, c);
-              lo[k] = Pack2<T>::pack((x - a) * kLoScale, (y - c) * kLoScale);
+              lo[k] = Pack2<T>::pack(fmaf(x - a, kLoScale, x * (kLoScale * 0x1p-24f)),
+                                     fmaf(y - c, kLoScale, y * (kLoScale * 0x1p-24f)));
             }
             ph[tl][c2] = make_uint4(hi[0], hi[1], hi[2], hi[3]);
             pl[tl][c2] = make_uint4(lo[0], lo[1], lo[2], lo[3]);

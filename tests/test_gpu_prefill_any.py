@@ -166,3 +166,24 @@ def test_weights_far_below_the_largest(device, q_dtype, D, gap):
     vc[at, 0] = 0
     check(device, q, kc, vc, table, lens, D)
     check(device, q, kc, vc, table, lens, D, causal=False)
+
+
+@pytest.mark.parametrize("q_dtype", [F32, F16, BF16])
+def test_infinite_values_stay_infinite(device, q_dtype):
+    """A value of +inf or -inf that every row sees, at dims of their own: infinite there, and the
+    finite result elsewhere (weights that the query type holds exactly among them: equal scores)."""
+    H, KVH, D, q_len, lens = 3, 1, 96, 127, [300]
+    for same in (False, True):
+        print(f"[case] infinite values {q_dtype} equal scores {same}", flush=True)
+        q, kc, vc, table = make(H, KVH, D, lens, q_len, q_dtype, q_dtype, 16, 7)
+        if same:
+            kc.zero_()
+        qd, kd, td, ld = (x.to(device) for x in (q, kc, table, torch.tensor(lens, dtype=torch.int32)))
+        assert kernel_route(qd, kd, td) == ROUTE
+        finite = paged_attention(qd, kd, vc.to(device), td, ld, causal=False)
+        at = int(table[0, 3])
+        vc[at, 5, 0, 10], vc[at, 6, 0, 11] = float("inf"), float("-inf")
+        out = paged_attention(qd, kd, vc.to(device), td, ld, causal=False)
+        assert bool((out[..., 10] == float("inf")).all()) and bool((out[..., 11] == float("-inf")).all())
+        keep = [d for d in range(D) if d not in (10, 11)]
+        assert torch.equal(out[..., keep], finite[..., keep])
