@@ -147,7 +147,9 @@ int msattn_paged_attention(const void* query, const void* k_cache, const void* v
  * least 0) are given and whose head dim is contiguous: a chunked prefill then reads a view,
  * such as a model's transposed projections (miniserve/model_runner.py:62-67), without a copy
  * made of it first. Same results. Calls that the two prefill kernels do not take return
- * MSATTN_ERR_UNSUPPORTED and launch nothing (the copying kernel needs 16-byte multiples).
+ * MSATTN_ERR_UNSUPPORTED and launch nothing; so do calls that run faster on an aligned copy: a
+ * query off 16 bytes, in its base or strides, whose copy would take the copying kernel or the
+ * any-layout kernel's vector loads.
  * The output must not overlap the query.
  */
 int msattn_paged_attention_strided(const void* query, int64_t q_batch_stride,

@@ -1084,8 +1084,8 @@ int choose_route(const void* query, const void* out, const void* k_cache, const 
 // msattn_paged_attention's body. `prefill_needs_ws`: whether the direct prefill route
 // checks the workspace size too (the workspace entry point's contract), although that
 // route does not touch it. `q_strides`: batch, token and head strides of a query that is not
-// contiguous, which the prefill kernels read in place; calls on other routes, and strides the
-// copying kernel's 16-byte loads cannot take, return MSATTN_ERR_UNSUPPORTED unlaunched.
+// contiguous, which the prefill kernels read in place; calls that a copy of the query runs
+// faster, and calls on other routes, return MSATTN_ERR_UNSUPPORTED unlaunched.
 int attention_impl(const void* query, const void* k_cache, const void* v_cache,
                    int64_t cache_block_stride, int64_t cache_slot_stride,
                    int64_t cache_head_stride, const int32_t* block_table,
@@ -1110,9 +1110,23 @@ int attention_impl(const void* query, const void* k_cache, const void* v_cache,
   const bool qs16 = (qs[0] * dtype_bytes(q_dtype)) % 16 == 0 &&
                     (qs[1] * dtype_bytes(q_dtype)) % 16 == 0 &&
                     (qs[2] * dtype_bytes(q_dtype)) % 16 == 0;
-  if (q_strides != nullptr && route != MSATTN_ROUTE_PREFILL_ANY &&
-      !(route == MSATTN_ROUTE_PREFILL && qs16))
-    return MSATTN_ERR_UNSUPPORTED;
+  if (q_strides != nullptr) {
+    if (route != MSATTN_ROUTE_PREFILL && route != MSATTN_ROUTE_PREFILL_ANY) return MSATTN_ERR_UNSUPPORTED;
+    // Off 16 bytes (base or strides) the query keeps the copying kernel and the vector loads of
+    // the whole any-layout launch out of reach, which an aligned copy would take: read in place
+    // only where such a copy takes neither (2 x 512 queries of H28/KVH4/D128 over 4.6k keys, base
+    // off by one element: 334 us in place, 78 copied; 256 of H24/KVH8/D96 55 and 36).
+    if (!qs16 || !aligned(query, 16)) {
+      const int copied = choose_route(nullptr, out, k_cache, v_cache, cache_block_stride,
+                                      cache_slot_stride, cache_head_stride, batch, q_len, num_heads,
+                                      num_kv_heads, head_dim, block_size, max_context, q_dtype,
+                                      kv_dtype, workspace_bytes);
+      const bool rows16 = cache_rows16(k_cache, v_cache, cache_block_stride, cache_slot_stride,
+                                       cache_head_stride, head_dim, kv_dtype);
+      if (copied != MSATTN_ROUTE_PREFILL_ANY || prefill_any_vec(nullptr, out, head_dim, rows16))
+        return MSATTN_ERR_UNSUPPORTED;
+    }
+  }
   if (route == MSATTN_ROUTE_PREFILL || route == MSATTN_ROUTE_PREFILL_ANY) {
     if (!query || !block_table || !context_lens || !workspace) return MSATTN_ERR_INVALID_ARG;
     if (!std::isfinite(scale)) return MSATTN_ERR_INVALID_ARG;

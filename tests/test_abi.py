@@ -323,6 +323,28 @@ def test_route_rejects_bad_arguments():
     assert lib.msattn_paged_attention_route(*bad, ctypes.byref(r)) == nat.ERR_INVALID_ARG
 
 
+@pytest.mark.parametrize("H,KVH,D,q_len,ctx,qd,bs,base,pad,in_place", [
+    (28, 4, 128, 512, 4608, nat.BF16, 16, 256, 8, True),    # the copying kernel: 16-byte multiples
+    (28, 4, 128, 512, 4608, nat.BF16, 16, 258, 8, False),   # base off 16 bytes
+    (28, 4, 128, 512, 4608, nat.BF16, 16, 256, 5, False),   # strides off
+    (24, 8, 96, 256, 2000, nat.BF16, 16, 256, 8, True),     # the any-layout kernel, vector loads
+    (24, 8, 96, 256, 2000, nat.BF16, 16, 258, 8, False),
+    (24, 8, 96, 256, 2000, nat.BF16, 16, 256, 5, False),
+    (28, 4, 128, 256, 4000, nat.F32, 16, 260, 4, False),
+    (24, 8, 90, 256, 20000, nat.BF16, 16, 258, 5, True),    # element loads either way
+    (14, 2, 64, 2, 500, nat.BF16, 16, 256, 8, False),       # the partition kernel: copied
+])
+def test_strided_query_read_in_place_or_copied(H, KVH, D, q_len, ctx, qd, bs, base, pad, in_place):
+    """A strided query is refused (for the caller to copy) where an aligned copy takes the copying
+    kernel or vector loads. No table is given: an accepted call ends as an invalid one."""
+    lib = nat.lib()
+    ws = lib.msattn_workspace_bytes(1, q_len, H, KVH, D, ctx)
+    st = lib.msattn_paged_attention_strided(
+        base, q_len * H * (D + pad), H * (D + pad), D + pad, 4096, 4096, bs * KVH * D, KVH * D, D, None,
+        512, 8192, 16384, ws, 1, q_len, H, KVH, D, bs, ctx, -(-ctx // bs), ctx, 1, 0, 0.1, qd, qd, None)
+    assert st == (nat.ERR_INVALID_ARG if in_place else nat.ERR_UNSUPPORTED)
+
+
 def test_append_rejects_bad_arguments():
     """msattn_paged_attention_append checks its pointers, types and geometry before it
     launches anything (these calls never reach a device)."""

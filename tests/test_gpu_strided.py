@@ -19,6 +19,9 @@ def views(x, pad=5):
     wide = x.new_zeros(B, T, H, D + pad)
     wide[..., :D] = x
     yield "padded", wide[..., :D]
+    flat = x.new_zeros(B, T, H * D + 8)
+    flat[..., 1:1 + H * D] = x.flatten(2)
+    yield "base off by an element", flat[..., 1:1 + H * D].unflatten(2, (H, D))
     yield "token-major", x.permute(1, 2, 0, 3).contiguous().permute(2, 0, 1, 3)
 
 
