@@ -1608,6 +1608,7 @@ int write_kv_impl(void* k_cache, void* v_cache, int64_t cache_block_stride,
     p.k_src[i] = (src_strides != nullptr ? src_strides : dense)[i];
     p.v_src[i] = (src_strides != nullptr ? src_strides : dense)[3 + i];
   }
+  p.dense = src_strides == nullptr ? 1 : 0;
   p.batch = batch;
   p.tokens = tokens;
   p.KVH = num_kv_heads;

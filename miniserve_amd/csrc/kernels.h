@@ -37,6 +37,7 @@ struct WriteKVParams {
   const int32_t* starts;
   int64_t blk_stride, slot_stride, head_stride;
   int64_t k_src[3], v_src[3];  // batch, token and head strides of k and v (elements)
+  int dense;                   // k and v are contiguous
   int batch, tokens, KVH, D, bs, num_blocks, W;
   int start_offset;  // added to starts[b] (-1: starts are context lengths after the append)
 };

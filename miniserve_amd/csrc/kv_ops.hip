@@ -18,14 +18,18 @@ __device__ __forceinline__ int64_t token_offset(const int32_t* table, int b, int
   return static_cast<int64_t>(phys) * blk_stride + static_cast<int64_t>(pos - pg * bs) * slot_stride;
 }
 
-// Element offset of (row b, token t, head h) in a source of strides s.
-__device__ __forceinline__ int64_t source_offset(const int64_t (&s)[3], int b, int t, int h) {
-  return b * s[0] + t * s[1] + h * s[2];
+// Element offset of dim d of (row b, token t, head h) in the source of strides s, which is
+// element `idx` of a contiguous one. DENSE is the kernels' parameter: the three 64-bit products
+// took 4 to 8 % of a contiguous write (2 x 16384 rows of 8 x 128, fp16 to fp8: 46.5 -> 50 us).
+template <bool DENSE>
+__device__ __forceinline__ int64_t source_offset(const int64_t (&s)[3], int b, int t, int h, int d,
+                                                 int64_t idx) {
+  return DENSE ? idx : b * s[0] + t * s[1] + h * s[2] + d;
 }
 
 // write_kv: cache[table[b, pos/bs], pos%bs, h, d] = convert(src[b, t, h, d]),
 // pos = starts[b] + t (miniserve/attention.py:111-133). One thread per element.
-template <typename ST, typename DT>
+template <typename ST, typename DT, bool DENSE>
 __global__ __launch_bounds__(kOpsThreads) void write_kv_kernel(const WriteKVParams p) {
   const int64_t total = static_cast<int64_t>(p.batch) * p.tokens * p.KVH * p.D;
   for (int64_t idx = static_cast<int64_t>(blockIdx.x) * kOpsThreads + threadIdx.x; idx < total;
@@ -41,14 +45,14 @@ __global__ __launch_bounds__(kOpsThreads) void write_kv_kernel(const WriteKVPara
     if (off < 0) continue;
     const int64_t dst = off + static_cast<int64_t>(h) * p.head_stride + d;
     Elt<DT>::store(static_cast<DT*>(p.k_cache) + dst,
-                   Elt<ST>::load(static_cast<const ST*>(p.k) + source_offset(p.k_src, b, t, h) + d));
+                   Elt<ST>::load(static_cast<const ST*>(p.k) + source_offset<DENSE>(p.k_src, b, t, h, d, idx)));
     Elt<DT>::store(static_cast<DT*>(p.v_cache) + dst,
-                   Elt<ST>::load(static_cast<const ST*>(p.v) + source_offset(p.v_src, b, t, h) + d));
+                   Elt<ST>::load(static_cast<const ST*>(p.v) + source_offset<DENSE>(p.v_src, b, t, h, d, idx)));
   }
 }
 
 // Same-dtype scatter: raw element copy (bit-exact, NaN payloads included).
-template <typename T>
+template <typename T, bool DENSE>
 __global__ __launch_bounds__(kOpsThreads) void write_kv_copy_kernel(const WriteKVParams p) {
   const int64_t total = static_cast<int64_t>(p.batch) * p.tokens * p.KVH * p.D;
   for (int64_t idx = static_cast<int64_t>(blockIdx.x) * kOpsThreads + threadIdx.x; idx < total;
@@ -63,8 +67,8 @@ __global__ __launch_bounds__(kOpsThreads) void write_kv_copy_kernel(const WriteK
                                      p.blk_stride, p.slot_stride);
     if (off < 0) continue;
     const int64_t dst = off + static_cast<int64_t>(h) * p.head_stride + d;
-    static_cast<T*>(p.k_cache)[dst] = static_cast<const T*>(p.k)[source_offset(p.k_src, b, t, h) + d];
-    static_cast<T*>(p.v_cache)[dst] = static_cast<const T*>(p.v)[source_offset(p.v_src, b, t, h) + d];
+    static_cast<T*>(p.k_cache)[dst] = static_cast<const T*>(p.k)[source_offset<DENSE>(p.k_src, b, t, h, d, idx)];
+    static_cast<T*>(p.v_cache)[dst] = static_cast<const T*>(p.v)[source_offset<DENSE>(p.v_src, b, t, h, d, idx)];
   }
 }
 
@@ -78,7 +82,7 @@ struct alignas(N) RawN {
   unsigned char b[N];
 };
 
-template <typename ST, typename DT, int E>
+template <typename ST, typename DT, int E, bool DENSE>
 __global__ __launch_bounds__(kOpsThreads) void write_kv_vec_kernel(const WriteKVParams p) {
   const int CPR = p.D / E;  // chunks per row
   const int64_t total = static_cast<int64_t>(p.batch) * p.tokens * p.KVH * CPR;
@@ -97,7 +101,7 @@ __global__ __launch_bounds__(kOpsThreads) void write_kv_vec_kernel(const WriteKV
 #pragma unroll
     for (int which = 0; which < 2; ++which) {
       const ST* sp = static_cast<const ST*>(which ? p.v : p.k) +
-                     source_offset(which ? p.v_src : p.k_src, b, t, h) + c * E;
+                     source_offset<DENSE>(which ? p.v_src : p.k_src, b, t, h, c * E, idx * E);
       DT* dp = static_cast<DT*>(which ? p.v_cache : p.k_cache) + dst;
       if constexpr (std::is_same<ST, DT>::value) {
         *reinterpret_cast<RawN<E * sizeof(ST)>*>(dp) =
@@ -136,44 +140,69 @@ static bool wkv_vec_ok(const WriteKVParams& p) {
          (p.head_stride * sizeof(DT)) % da == 0;
 }
 
-template <typename ST, typename DT>
+template <typename ST, typename DT, bool DENSE>
 static hipError_t launch_wkv(const WriteKVParams& p, hipStream_t stream) {
   constexpr int E = sizeof(ST) >= 4 || sizeof(DT) >= 4 ? 4 : 8;
   if (wkv_vec_ok<ST, DT, E>(p)) {
     const int64_t total = static_cast<int64_t>(p.batch) * p.tokens * p.KVH * (p.D / E);
-    hipLaunchKernelGGL((write_kv_vec_kernel<ST, DT, E>), dim3(grid_for(total)), dim3(kOpsThreads),
-                       0, stream, p);
+    hipLaunchKernelGGL((write_kv_vec_kernel<ST, DT, E, DENSE>), dim3(grid_for(total)),
+                       dim3(kOpsThreads), 0, stream, p);
     return hipGetLastError();
   }
   const int64_t total = static_cast<int64_t>(p.batch) * p.tokens * p.KVH * p.D;
-  hipLaunchKernelGGL((write_kv_kernel<ST, DT>), dim3(grid_for(total)), dim3(kOpsThreads), 0,
+  hipLaunchKernelGGL((write_kv_kernel<ST, DT, DENSE>), dim3(grid_for(total)), dim3(kOpsThreads), 0,
                      stream, p);
   return hipGetLastError();
 }
 
-template <typename T>
+template <typename T, bool DENSE>
 static hipError_t launch_wkv_copy(const WriteKVParams& p, hipStream_t stream) {
   constexpr int E = 16 / sizeof(T);
   if (wkv_vec_ok<T, T, E>(p)) {
     const int64_t total = static_cast<int64_t>(p.batch) * p.tokens * p.KVH * (p.D / E);
-    hipLaunchKernelGGL((write_kv_vec_kernel<T, T, E>), dim3(grid_for(total)), dim3(kOpsThreads),
-                       0, stream, p);
+    hipLaunchKernelGGL((write_kv_vec_kernel<T, T, E, DENSE>), dim3(grid_for(total)),
+                       dim3(kOpsThreads), 0, stream, p);
     return hipGetLastError();
   }
   const int64_t total = static_cast<int64_t>(p.batch) * p.tokens * p.KVH * p.D;
-  hipLaunchKernelGGL(write_kv_copy_kernel<T>, dim3(grid_for(total)), dim3(kOpsThreads), 0, stream,
-                     p);
+  hipLaunchKernelGGL((write_kv_copy_kernel<T, DENSE>), dim3(grid_for(total)), dim3(kOpsThreads), 0,
+                     stream, p);
   return hipGetLastError();
 }
 
-template <typename ST>
+template <typename ST, bool DENSE>
 static hipError_t launch_wkv_src(const WriteKVParams& p, int dst_dtype, hipStream_t stream,
                                  bool* supported) {
   switch (dst_dtype) {
-    case 0: return launch_wkv<ST, float>(p, stream);
-    case 1: return launch_wkv<ST, _Float16>(p, stream);
-    case 2: return launch_wkv<ST, bf16_t>(p, stream);
-    case 3: return launch_wkv<ST, fp8_t>(p, stream);
+    case 0: return launch_wkv<ST, float, DENSE>(p, stream);
+    case 1: return launch_wkv<ST, _Float16, DENSE>(p, stream);
+    case 2: return launch_wkv<ST, bf16_t, DENSE>(p, stream);
+    case 3: return launch_wkv<ST, fp8_t, DENSE>(p, stream);
+    default: break;
+  }
+  *supported = false;
+  return hipSuccess;
+}
+
+template <bool DENSE>
+static hipError_t launch_wkv_types(const WriteKVParams& p, int src_dtype, int dst_dtype,
+                                   hipStream_t stream, bool* supported) {
+  *supported = true;
+  if (src_dtype == dst_dtype) {
+    switch (src_dtype) {
+      case 0: return launch_wkv_copy<uint32_t, DENSE>(p, stream);
+      case 1:
+      case 2: return launch_wkv_copy<uint16_t, DENSE>(p, stream);
+      case 3: return launch_wkv_copy<uint8_t, DENSE>(p, stream);
+      default: break;
+    }
+    *supported = false;
+    return hipSuccess;
+  }
+  switch (src_dtype) {
+    case 0: return launch_wkv_src<float, DENSE>(p, dst_dtype, stream, supported);
+    case 1: return launch_wkv_src<_Float16, DENSE>(p, dst_dtype, stream, supported);
+    case 2: return launch_wkv_src<bf16_t, DENSE>(p, dst_dtype, stream, supported);
     default: break;
   }
   *supported = false;
@@ -182,26 +211,8 @@ static hipError_t launch_wkv_src(const WriteKVParams& p, int dst_dtype, hipStrea
 
 hipError_t launch_write_kv(const WriteKVParams& p, int src_dtype, int dst_dtype,
                            hipStream_t stream, bool* supported) {
-  *supported = true;
-  if (src_dtype == dst_dtype) {
-    switch (src_dtype) {
-      case 0: return launch_wkv_copy<uint32_t>(p, stream);
-      case 1:
-      case 2: return launch_wkv_copy<uint16_t>(p, stream);
-      case 3: return launch_wkv_copy<uint8_t>(p, stream);
-      default: break;
-    }
-    *supported = false;
-    return hipSuccess;
-  }
-  switch (src_dtype) {
-    case 0: return launch_wkv_src<float>(p, dst_dtype, stream, supported);
-    case 1: return launch_wkv_src<_Float16>(p, dst_dtype, stream, supported);
-    case 2: return launch_wkv_src<bf16_t>(p, dst_dtype, stream, supported);
-    default: break;
-  }
-  *supported = false;
-  return hipSuccess;
+  return p.dense ? launch_wkv_types<true>(p, src_dtype, dst_dtype, stream, supported)
+                 : launch_wkv_types<false>(p, src_dtype, dst_dtype, stream, supported);
 }
 
 // Gather: out[b, pos, h, d] = cache[blk, pos % bs, h, d] with blk = table[b, pos / bs]
