@@ -72,6 +72,20 @@ def _readable_in_place(t: torch.Tensor, *written: torch.Tensor | None) -> bool:
         all(w is None or w.untyped_storage().data_ptr() != base for w in written)
 
 
+# Elements of a source off 16 bytes up to which write_kv reads it in place, element by element,
+# rather than a copy of it in 16-byte chunks: measured 2.8 against 7.6 us at 0.1 M elements
+# (fp16 rows of 8 x 128), level at 3 M, 44 against 30 at 8 M (fp32 level at 6 M, 45 and 43 at 8 M).
+_ELEMENT_READS_MAX = 3 << 20
+
+
+def _worth_in_place(t: torch.Tensor) -> bool:
+    """Whether write_kv reads `t` through its strides at least as fast as a copy of it: in 16-byte
+    chunks, where a copy would not make chunks of it either, or where it is small."""
+    es = t.element_size()
+    return t.numel() <= _ELEMENT_READS_MAX or (t.shape[3] * es) % 16 != 0 or \
+        (t.data_ptr() % 16 == 0 and all(st * es % 16 == 0 for st in t.stride()[:3]))
+
+
 def _require_gpu(t: torch.Tensor, what: str) -> None:
     if t.device.type != "cuda":
         raise RuntimeError(
@@ -251,7 +265,8 @@ class PagedAttention:
             raise ValueError("start needs one entry per batch row")
         starts = starts.contiguous()
         if not (k.is_contiguous() and v.is_contiguous()) and \
-                _readable_in_place(k, k_cache, v_cache) and _readable_in_place(v, k_cache, v_cache):
+                _readable_in_place(k, k_cache, v_cache) and \
+                _readable_in_place(v, k_cache, v_cache) and _worth_in_place(k) and _worth_in_place(v):
             # views, such as a model's transposed projections, are read where they lie
             status = nat.lib().msattn_write_kv_strided(
                 k_cache.data_ptr(), v_cache.data_ptr(), k_cache.stride(0), k_cache.stride(1),

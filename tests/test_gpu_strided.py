@@ -87,3 +87,27 @@ def test_write_kv_from_the_cache_itself(device):
     pa.write_kv(kc, vc, k, v, table, start=1)
     assert torch.equal(kc.view(1, 128, 2, 64)[:, 1:31], want[0])
     assert torch.equal(vc.view(1, 128, 2, 64)[:, 1:31], want[1])
+
+
+@pytest.mark.parametrize("T,name,in_place", [
+    (3072, "base off by an element", True), (3073, "base off by an element", False),
+    (3073, "transposed", True), (3073, "padded", False)])
+def test_large_sources_off_16_bytes_are_copied(device, monkeypatch, T, name, in_place):
+    """Rows of 8 x 128 past the line take the vector kernel over a copy unless their strides do."""
+    from miniserve_amd import _native as nat
+
+    pa = PagedAttention(8, 8, 128, num_blocks=T // 16 + 1, block_size=16, dtype=F16, kv_dtype=F16,
+                        device=device)
+    k, v = (torch.randn(1, T, 8, 128, device=device).to(F16) for _ in range(2))
+    table = torch.randperm(T // 16 + 1, device=device).to(torch.int32)[None]
+    want = pa.allocate_kv_cache()
+    pa.write_kv(*want, k, v, table)
+    kv = dict(views(k))[name]
+    calls = []
+    strided = nat.lib().msattn_write_kv_strided
+    monkeypatch.setattr(nat.lib(), "msattn_write_kv_strided",
+                        lambda *a: calls.append(1) or strided(*a))
+    got = pa.allocate_kv_cache()
+    pa.write_kv(*got, kv, v, table)
+    assert bool(calls) == in_place
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
