@@ -113,8 +113,9 @@ size_t msattn_workspace_bytes(int batch, int q_len, int num_heads, int num_kv_he
  * page sizes and alignments) runs on the any-layout prefill kernel where a cost model in
  * sizes prefers it, writing the output directly (or through a fold launch), else on the
  * partition kernel (an fp32 query) or the generic kernel, which needs only element-aligned
- * caches. msattn_paged_attention_route names the route; it has no window argument, and a
- * windowed decode is routed by what its window shows, not by its table.
+ * caches. msattn_paged_attention_route names the route, and
+ * msattn_paged_attention_route_window that of a call under a window, whose decodes are routed by
+ * what the window shows.
  * Runs msattn_paged_attention_partials followed by msattn_merge_partials, except:
  * chunked prefill on the MFMA kernel (bf16/fp16 query 16-byte aligned, output 8-byte
  * aligned, cache of the query's type, fp8 e4m3 or fp32, head_dim 64 or 128, more than 16
@@ -205,6 +206,15 @@ int msattn_paged_attention_route(const void* query, const void* out, const void*
                                  int q_len, int num_heads, int num_kv_heads, int head_dim,
                                  int block_size, int max_context, int q_dtype, int kv_dtype,
                                  size_t workspace_bytes, int* route);
+
+/* msattn_paged_attention_route for a call under a sliding window (window <= 0: none). */
+int msattn_paged_attention_route_window(const void* query, const void* out, const void* k_cache,
+                                        const void* v_cache, int64_t cache_block_stride,
+                                        int64_t cache_slot_stride, int64_t cache_head_stride,
+                                        int batch, int q_len, int num_heads, int num_kv_heads,
+                                        int head_dim, int block_size, int max_context, int window,
+                                        int q_dtype, int kv_dtype, size_t workspace_bytes,
+                                        int* route);
 
 /*
  * msattn_paged_attention for decode (q_len == 1) with rotate-half RoPE applied to

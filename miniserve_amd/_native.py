@@ -57,6 +57,9 @@ SIGNATURES = {
     "msattn_paged_attention_route": (c_int, [
         c_vp, c_vp, c_vp, c_vp, c_i64, c_i64, c_i64, c_int, c_int, c_int, c_int, c_int, c_int,
         c_int, c_int, c_int, c_size, ctypes.POINTER(c_int)]),
+    "msattn_paged_attention_route_window": (c_int, [
+        c_vp, c_vp, c_vp, c_vp, c_i64, c_i64, c_i64, c_int, c_int, c_int, c_int, c_int, c_int,
+        c_int, c_int, c_int, c_int, c_size, ctypes.POINTER(c_int)]),
     "msattn_paged_attention_rope": (c_int, [
         c_vp, c_vp, c_vp, c_i64, c_i64, c_i64, c_vp, c_vp, c_vp, c_vp, c_size,
         c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int,

@@ -559,10 +559,11 @@ def paged_attention_append(query: torch.Tensor, k_new: torch.Tensor, v_new: torc
 
 def kernel_route(query: torch.Tensor, k_cache: torch.Tensor, block_table,
                  max_context: int | None = None, out: torch.Tensor | None = None,
-                 workspace_bytes: int | None = None) -> str:
+                 workspace_bytes: int | None = None, window: int | None = None) -> str:
     """Name of the kernel ``paged_attention`` runs for this call: "prefill", "prefill
-    stream-K" (the prefill kernel's stream-K schedule), "partition-fused", "partition",
-    "stream-K" (the stream-K decode kernel) or "generic" (msattn_paged_attention_route).
+    stream-K" (the prefill kernel's stream-K schedule), "prefill any-layout",
+    "partition-fused", "partition", "stream-K" (the stream-K decode kernel) or "generic"
+    (msattn_paged_attention_route_window).
 
     The choice depends on shapes, types and alignment, not on context-length values;
     ``max_context`` defaults to the table capacity, ``workspace_bytes`` to the call's own
@@ -580,10 +581,10 @@ def kernel_route(query: torch.Tensor, k_cache: torch.Tensor, block_table,
     q = query if query.is_contiguous() else query.contiguous()
     out_ptr = out.data_ptr() if out is not None else q.data_ptr()
     r = ctypes.c_int(0)
-    nat.check("msattn_paged_attention_route", lib.msattn_paged_attention_route(
+    nat.check("msattn_paged_attention_route_window", lib.msattn_paged_attention_route_window(
         q.data_ptr(), out_ptr, k_cache.data_ptr(), k_cache.data_ptr(), k_cache.stride(0),
         k_cache.stride(1), k_cache.stride(2), B, q_len, H, KVH, D, bs, max_context,
-        nat.dtype_code(query.dtype), nat.dtype_code(k_cache.dtype), workspace_bytes,
+        int(window or 0), nat.dtype_code(query.dtype), nat.dtype_code(k_cache.dtype), workspace_bytes,
         ctypes.byref(r)))
     return nat.ROUTE_NAMES[r.value]
 

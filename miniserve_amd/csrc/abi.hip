@@ -1055,7 +1055,7 @@ bool prefill_any_preferred(int batch, int q_len, int num_heads, int num_kv_heads
 int choose_route(const void* query, const void* out, const void* k_cache, const void* v_cache,
                  int64_t cache_block_stride, int64_t cache_slot_stride, int64_t cache_head_stride,
                  int batch, int q_len, int num_heads, int num_kv_heads, int head_dim,
-                 int block_size, int max_context, int q_dtype, int kv_dtype,
+                 int block_size, int max_context, int window, int q_dtype, int kv_dtype,
                  size_t workspace_bytes) {
   const bool rows16 = cache_rows16(k_cache, v_cache, cache_block_stride, cache_slot_stride,
                                    cache_head_stride, head_dim, kv_dtype);
@@ -1075,7 +1075,7 @@ int choose_route(const void* query, const void* out, const void* k_cache, const 
     return MSATTN_ROUTE_PREFILL_ANY;
   const PartialsPlan pl =
       plan_partials(query, q_dtype, kv_dtype, head_dim, block_size, cache_slot_stride, rows16,
-                    batch, q_len, num_heads, num_kv_heads, max_context, true, 0, 0);
+                    batch, q_len, num_heads, num_kv_heads, max_context, true, 0, window);
   if (pl.kind == 1) return MSATTN_ROUTE_STREAMK;
   if (pl.kind == 2) return MSATTN_ROUTE_PARTITION_FUSED;
   return pl.use_mfma ? MSATTN_ROUTE_PARTITION : MSATTN_ROUTE_GENERIC;
@@ -1102,8 +1102,8 @@ int attention_impl(const void* query, const void* k_cache, const void* v_cache,
     return MSATTN_ERR_INVALID_ARG;
   const int route = choose_route(query, out, k_cache, v_cache, cache_block_stride,
                                  cache_slot_stride, cache_head_stride, batch, q_len, num_heads,
-                                 num_kv_heads, head_dim, block_size, max_context, q_dtype, kv_dtype,
-                                 workspace_bytes);
+                                 num_kv_heads, head_dim, block_size, max_context, window, q_dtype,
+                                 kv_dtype, workspace_bytes);
   const int64_t q_row = head_dim, q_tok = q_row * num_heads;
   const int64_t dense_q[3] = {q_tok * q_len, q_tok, q_row};
   const int64_t* const qs = q_strides != nullptr ? q_strides : dense_q;
@@ -1119,8 +1119,8 @@ int attention_impl(const void* query, const void* k_cache, const void* v_cache,
     if (!qs16 || !aligned(query, 16)) {
       const int copied = choose_route(nullptr, out, k_cache, v_cache, cache_block_stride,
                                       cache_slot_stride, cache_head_stride, batch, q_len, num_heads,
-                                      num_kv_heads, head_dim, block_size, max_context, q_dtype,
-                                      kv_dtype, workspace_bytes);
+                                      num_kv_heads, head_dim, block_size, max_context, window,
+                                      q_dtype, kv_dtype, workspace_bytes);
       const bool rows16 = cache_rows16(k_cache, v_cache, cache_block_stride, cache_slot_stride,
                                        cache_head_stride, head_dim, kv_dtype);
       if (copied != MSATTN_ROUTE_PREFILL_ANY || prefill_any_vec(nullptr, out, head_dim, rows16))
@@ -1321,7 +1321,7 @@ int msattn_paged_attention_noalloc(const void* query, const void* k_cache, const
   // kernel can run there (it uses no scratch); any other call past the scratch is refused.
   if (choose_route(query, out, k_cache, v_cache, cache_block_stride, cache_slot_stride,
                    cache_head_stride, batch, q_len, num_heads, num_kv_heads, head_dim, block_size,
-                   max_context, q_dtype, kv_dtype, kScratchBytes) != MSATTN_ROUTE_PREFILL) {
+                   max_context, window, q_dtype, kv_dtype, kScratchBytes) != MSATTN_ROUTE_PREFILL) {
     const Layout L = workspace_layout(batch, q_len, num_heads, num_kv_heads, head_dim, max_context);
     if (L.total() > kScratchBytes) return MSATTN_ERR_WORKSPACE;
   }
@@ -1341,6 +1341,19 @@ int msattn_paged_attention_route(const void* query, const void* out, const void*
                                  int q_len, int num_heads, int num_kv_heads, int head_dim,
                                  int block_size, int max_context, int q_dtype, int kv_dtype,
                                  size_t workspace_bytes, int* route) {
+  return msattn_paged_attention_route_window(
+      query, out, k_cache, v_cache, cache_block_stride, cache_slot_stride, cache_head_stride, batch,
+      q_len, num_heads, num_kv_heads, head_dim, block_size, max_context, 0, q_dtype, kv_dtype,
+      workspace_bytes, route);
+}
+
+int msattn_paged_attention_route_window(const void* query, const void* out, const void* k_cache,
+                                        const void* v_cache, int64_t cache_block_stride,
+                                        int64_t cache_slot_stride, int64_t cache_head_stride,
+                                        int batch, int q_len, int num_heads, int num_kv_heads,
+                                        int head_dim, int block_size, int max_context, int window,
+                                        int q_dtype, int kv_dtype, size_t workspace_bytes,
+                                        int* route) {
   if (!route) return MSATTN_ERR_INVALID_ARG;
   *route = 0;
   if (!geometry_ok(batch, q_len, num_heads, num_kv_heads, head_dim, max_context))
@@ -1351,7 +1364,7 @@ int msattn_paged_attention_route(const void* query, const void* out, const void*
     return MSATTN_ERR_INVALID_ARG;
   const int r = choose_route(query, out, k_cache, v_cache, cache_block_stride, cache_slot_stride,
                              cache_head_stride, batch, q_len, num_heads, num_kv_heads, head_dim,
-                             block_size, max_context, q_dtype, kv_dtype, workspace_bytes);
+                             block_size, max_context, window, q_dtype, kv_dtype, workspace_bytes);
   if (r != MSATTN_ROUTE_PREFILL &&
       workspace_bytes < workspace_layout(batch, q_len, num_heads, num_kv_heads, head_dim,
                                          max_context).total())

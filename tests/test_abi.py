@@ -230,14 +230,19 @@ def test_noalloc_entry_checks_before_any_hip_call():
 # ------------------------------------------------------------------ kernel routes
 
 def route(B, q_len, H, KVH, D, ctx, qd=nat.BF16, kvd=None, ws=None, slot_stride=None,
-          bs=16, query=256, out=256):
-    """msattn_paged_attention_route for a contiguous cache [.., bs, KVH, D] (or the given
+          bs=16, query=256, out=256, window=None):
+    """msattn_paged_attention_route (or, given a window, its form for one) for a contiguous cache [.., bs, KVH, D] (or the given
     slot stride), with the call's own workspace size unless `ws` is given."""
     lib = nat.lib()
     kvd = qd if kvd is None else kvd
     ss = KVH * D if slot_stride is None else slot_stride
     ws = lib.msattn_workspace_bytes(B, q_len, H, KVH, D, ctx) if ws is None else ws
     r = ctypes.c_int(-1)
+    if window is not None:
+        st = lib.msattn_paged_attention_route_window(
+            query, out, 256, 256, bs * ss, ss, D, B, q_len, H, KVH, D, bs, ctx, window, qd, kvd, ws,
+            ctypes.byref(r))
+        return st, r.value
     st = lib.msattn_paged_attention_route(query, out, 256, 256, bs * ss, ss, D, B, q_len, H, KVH,
                                           D, bs, ctx, qd, kvd, ws, ctypes.byref(r))
     return st, r.value
@@ -272,6 +277,22 @@ def test_route_policy(shape, want):
     head) pairs to fill the device, stream-K scheduled where the cost model prefers it
     (sizes from the measured prefill sweep)."""
     st, r = route(*shape)
+    assert st == nat.OK and r == want, (nat.ROUTE_NAMES.get(r), shape)
+
+
+@pytest.mark.parametrize("shape,kv,window,want", [
+    ((32, 1, 28, 4, 128, 6144), nat.FP8_E4M3, 0, nat.ROUTE_PARTITION_FUSED),   # 49,152 table tiles
+    ((32, 1, 28, 4, 128, 6144), nat.FP8_E4M3, 4096, nat.ROUTE_STREAMK),        # 32,768 shown
+    ((32, 1, 28, 4, 128, 6144), nat.FP8_E4M3, 4080, nat.ROUTE_PARTITION_FUSED),
+    ((32, 1, 28, 4, 128, 6144), nat.FP8_E4M3, 6144, nat.ROUTE_PARTITION_FUSED),  # hides nothing
+    ((64, 1, 32, 8, 128, 8192), nat.BF16, 1024, nat.ROUTE_PARTITION_FUSED),
+    ((64, 1, 32, 8, 128, 8192), nat.BF16, 8192, nat.ROUTE_STREAMK),
+    ((64, 1, 32, 8, 128, 8192), nat.BF16, 1 << 30, nat.ROUTE_STREAMK),
+    ((2, 512, 28, 4, 128, 4608), nat.BF16, 100, nat.ROUTE_PREFILL),
+])
+def test_route_under_a_window(shape, kv, window, want):
+    """A windowed decode's route: by the tiles its window shows, the table's if it hides none."""
+    st, r = route(*shape, kvd=kv, window=window)
     assert st == nat.OK and r == want, (nat.ROUTE_NAMES.get(r), shape)
 
 

@@ -64,14 +64,17 @@ CASES = {
                                                  torch.float8_e4m3fn, 16, 512, 0, "stream-K"),
     "stream-K table, bf16 over fp32": (32, 8, 128, torch.bfloat16, torch.float32, 16, 512, 0,
                                        "stream-K"),
+    # the partition kernel under a window that shows few of a stream-K table's tiles
     "stream-K table, fp16 D64 G7 window": (14, 2, 64, torch.float16, torch.float16, 64, 1024,
-                                           1000, "stream-K"),
+                                           1000, "partition-fused"),
+    "fp16 D64 G7, stream-K window": (14, 2, 64, torch.float16, torch.float16, 64, 1024, 12288,
+                                     "stream-K"),
     # a window that shows enough tiles for stream-K, whose kernel has no append over fp8, over a
     # table below that line without the window (two launches)
     "fp8 G7 D128, window at the stream-K line": (28, 4, 128, torch.bfloat16, torch.float8_e4m3fn,
-                                                 32, 384, 4096, "partition-fused"),
+                                                 32, 384, 4096, "stream-K"),
     "fp8 G7 D64, window at the stream-K line": (14, 2, 64, torch.bfloat16, torch.float8_e4m3fn,
-                                                64, 384, 4096, "partition-fused"),
+                                                64, 384, 4096, "stream-K"),
     # a window that shows a stream-K launch over a 16-bit cache: the append in that launch
     "bf16 window, stream-K": (32, 8, 128, torch.bfloat16, torch.bfloat16, 64, 160, 2100,
                               "stream-K"),
@@ -80,9 +83,8 @@ CASES = {
 }
 
 
-# The kind word of the workspace header after the call (1 stream-K, 2 the partition kernel).
-KIND = {"fp8 G7 D128, window at the stream-K line": 1, "fp8 G7 D64, window at the stream-K line": 1,
-        "bf16 window, stream-K": 1}
+# The workspace header's kind word as each kernel leaves it.
+KIND = {"stream-K": 1, "partition-fused": 2, "generic": 0}
 
 
 @pytest.mark.parametrize("name", list(CASES))
@@ -110,14 +112,14 @@ def test_append_equals_write_kv_then_decode(device, name):
         vn = torch.randn(B, 1, KVH, D, generator=gd, device=device).to(q_dtype)
         td = tab.to(device)
         ld = torch.tensor(lens, dtype=torch.int32, device=device)
-        assert kernel_route(q, kc_a, td, max_context=cap) == route
+        assert kernel_route(q, kc_a, td, max_context=cap, window=window or None) == route
         write_kv_ref(kc_b, vc_b, kn, vn, td, ld)
         ref = paged_attention(q, kc_b, vc_b, td, ld, max_context=cap,
                               window=window or None)
         out = paged_attention_append(q, kn, vn, kc_a, vc_a, td, ld, max_context=cap,
                                      window=window or None, workspace=ws)
         torch.cuda.synchronize()
-        assert KIND.get(name, int(ws[:4].view(torch.int32))) == int(ws[:4].view(torch.int32))
+        assert int(ws[:4].view(torch.int32)) == KIND[route]
         assert torch.equal(kc_a.view(torch.uint8), kc_b.view(torch.uint8)), "K caches differ"
         assert torch.equal(vc_a.view(torch.uint8), vc_b.view(torch.uint8)), "V caches differ"
         assert not torch.isnan(out.float()).any()
