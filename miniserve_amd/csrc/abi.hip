@@ -533,6 +533,12 @@ struct PartialsPlan {
   int kind;
 };
 
+// A window as long as any context hides nothing: none, so that such a call takes the routes and
+// shapes of one without and no kernel adds to a window near 2^31.
+int effective_window(int window, int max_context) {
+  return window > 0 && window < max_context ? window : 0;
+}
+
 // Whether a sliding window's size, not the table's, sets a decode's route and partitions. Not
 // over an fp8 cache at 4 rows per tile and head_dim 128, whose widening work wants the long
 // runs of stream-K and of the wide shape: 64 x H32/KVH8 under a 1024-token window 33.5 us
@@ -576,8 +582,9 @@ PartialsPlan plan_partials(const void* query, int q_dtype, int kv_dtype, int hea
   // A sliding window counts for what it shows: 32 sequences of 16k tokens under a 1024-token
   // window (H32/KVH8/D128 fp16) take 30.9 us on stream-K and the merge, 27.7 on the partition
   // kernel; 64 under a 128-token one 22.1 and 17.6.
-  const bool windowed = merges && windows_shrink(kv_dtype == MSATTN_FP8_E4M3, pl.RT, head_dim, window) &&
-                        window < max_context;
+  window = effective_window(window, max_context);
+  const bool windowed =
+      merges && windows_shrink(kv_dtype == MSATTN_FP8_E4M3, pl.RT, head_dim, window);
   const int seen = windowed ? window : max_context;
   const int64_t tile_capacity = static_cast<int64_t>(batch) * num_kv_heads * ceil_div(seen, 16);
   const bool kv_fp8 = kv_dtype == MSATTN_FP8_E4M3;
@@ -666,7 +673,7 @@ int partials_impl(const void* query, const void* k_cache, const void* v_cache,
   p.max_parts = L.max_parts;
   p.part = L.part;
   p.causal = causal ? 1 : 0;
-  p.window = window > 0 ? window : 0;
+  p.window = effective_window(window, max_context);
   p.scale_log2 = scale * kLog2e;
   p.rows_per_kvh = rows;
   p.rtiles = ceil_div(rows, RT);
@@ -1159,7 +1166,7 @@ int attention_impl(const void* query, const void* k_cache, const void* v_cache,
     pp.W = table_width;
     pp.max_ctx = max_context;
     pp.causal = causal ? 1 : 0;
-    pp.window = window > 0 ? window : 0;
+    pp.window = effective_window(window, max_context);
     pp.scale_log2 = scale * kLog2e;
     pp.rows_per_kvh = q_len * pp.G;
     pp.rblocks = ceil_div(pp.rows_per_kvh, kPfRows);

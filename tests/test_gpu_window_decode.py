@@ -122,3 +122,26 @@ def test_window_tiles_that_take_stream_k(device, H, KVH, D, B, window, q_dtype, 
                                     window=window, kv_cast=True)
     err = np.abs(out[:3].double().cpu().numpy() - ref).max()
     assert err < (1e-4 if q_dtype == torch.float32 else 2e-2 * np.abs(ref).max())
+
+
+@pytest.mark.parametrize("window", [96, 1 << 20, 2 ** 31 - 1])
+@pytest.mark.parametrize("H,KVH,D,q_len,q_dtype,kv_dtype,pages", [
+    (4, 4, 64, 16, torch.bfloat16, torch.bfloat16, 6),        # the partition kernel
+    (28, 4, 128, 1, torch.bfloat16, torch.bfloat16, 6),
+    (28, 4, 128, 60, torch.bfloat16, torch.float8_e4m3fn, 6),  # chunks on both prefill kernels
+    (6, 2, 96, 60, torch.float32, torch.float32, 4096),
+    (6, 2, 96, 2, torch.float32, torch.float32, 6),           # the generic kernel
+])
+def test_a_window_that_hides_nothing(device, H, KVH, D, q_len, q_dtype, kv_dtype, pages, window):
+    """Contexts shorter than the chunk among them: bit for bit the call without a window, up to
+    the largest value that a window can take."""
+    cap = 16 * pages
+    window = max(window, cap)
+    print(f"[case] H={H}/{KVH} D={D} q_len={q_len} {q_dtype}/{kv_dtype} window={window}", flush=True)
+    g = torch.Generator().manual_seed(q_len)
+    lens = torch.tensor([5, 0, 96, 61], dtype=torch.int32, device=device)
+    q = torch.randn(4, q_len, H, D, generator=g).to(q_dtype).to(device)
+    kc, vc = (torch.randn(32, 16, KVH, D, generator=g).to(kv_dtype).to(device) for _ in range(2))
+    table = torch.randint(0, 32, (4, pages), generator=g).to(torch.int32).to(device)
+    want = paged_attention(q, kc, vc, table, lens)
+    assert torch.equal(paged_attention(q, kc, vc, table, lens, window=window), want)
