@@ -64,12 +64,19 @@ def apply_rope(q: torch.Tensor, k: torch.Tensor | None, cos: torch.Tensor, sin: 
     return q_rot, k_rot
 
 
+def _span(t: torch.Tensor) -> tuple[int, int]:
+    """First byte of a tensor's storage and the one past its last."""
+    storage = t.untyped_storage()
+    return storage.data_ptr(), storage.data_ptr() + storage.nbytes()
+
+
 def _readable_in_place(t: torch.Tensor, *written: torch.Tensor | None) -> bool:
     """Whether a kernel may read `t` [batch, tokens, heads, dim] through its strides: rows of
-    contiguous dims, in memory that none of the tensors the call writes shares."""
-    base = t.untyped_storage().data_ptr()
+    contiguous dims, in memory that none of the tensors the call writes shares (two storages may
+    lie in one allocation: a tensor taken from DLPack has one of its own)."""
+    lo, hi = _span(t)
     return t.stride(3) == 1 and t.numel() > 0 and not t.is_neg() and \
-        all(w is None or w.untyped_storage().data_ptr() != base for w in written)
+        all(w is None or _span(w)[1] <= lo or hi <= _span(w)[0] for w in written)
 
 
 # Elements of a source off 16 bytes up to which write_kv reads it in place, element by element,

@@ -165,3 +165,20 @@ def test_runner_table_fill_matches_row_by_row():
         fill_table(np.zeros((2, 3), dtype=np.int32), [[1, 2, 3, 4]], 1)
     with pytest.raises(ValueError):
         fill_table(np.zeros((2, 3), dtype=np.int32), [[1]], 2)
+
+
+def test_views_read_in_place_share_no_memory_with_what_is_written():
+    """A view is read through its strides only where no written tensor lies in its memory, also
+    by a storage of its own (DLPack)."""
+    from miniserve_amd.attention import _readable_in_place
+
+    cache = torch.zeros(8, 16, 2, 64)
+    view = cache.view(1, 128, 2, 64)[:, 1:61:2]
+    other = torch.zeros(1, 2, 30, 64).transpose(1, 2)
+    alias = torch.from_dlpack(view)
+    assert alias.untyped_storage().data_ptr() != cache.untyped_storage().data_ptr()
+    assert _readable_in_place(other, cache, None)
+    assert not _readable_in_place(view, cache)
+    assert not _readable_in_place(alias, cache)
+    assert not _readable_in_place(view, None, alias)
+    assert not _readable_in_place(other.transpose(2, 3), cache)  # strided dims
