@@ -43,7 +43,7 @@ def make(H, KVH, D, lens, q_len, q_dtype, kv_dtype, bs, seed, pad=0):
     return q, caches[0], caches[1], table
 
 
-def check(device, q, kc, vc, table, lens, D, *, causal=True, window=None, scale=None):
+def check(device, q, kc, vc, table, lens, D, *, causal=True, window=None, scale=None, shares=None):
     qd, kd, vd, td = (x.to(device) for x in (q, kc, vc, table))
     kd, vd = kd[..., :D], vd[..., :D]
     ln = torch.tensor(lens, dtype=torch.int32, device=device)
@@ -56,6 +56,10 @@ def check(device, q, kc, vc, table, lens, D, *, causal=True, window=None, scale=
     torch.cuda.synchronize()
     assert torch.equal(outs[0], outs[1])
     assert not ws[:(64 + 4096) * 4].view(torch.int32)[64:].any(), "tickets not at zero"
+    if shares is not None:  # a launch of shares leaves its work list behind the tickets
+        tasks = -(-q.shape[1] * q.shape[2] // kc.shape[2] // 128) * kc.shape[2] * q.shape[0]
+        work_list = ws[(64 + 4096) * 4:(64 + 4096 + tasks + 2) * 4].view(torch.int32)
+        assert bool(work_list.any()) == shares
     ref = dense.paged_attention_f64(q, kc[..., :D], vc[..., :D], table.long(), lens, causal=causal,
                                     window=window, kv_cast=True,
                                     **({} if scale is None else {"scale": scale}))
@@ -97,7 +101,7 @@ def test_layouts(device, q_dtype, kv_dtype, H, KVH, D, bs, pad):
     table[0, 1] = -1
     table[0, 9] = 10 ** 6
     holed = paged_attention(q.to(device), kc.to(device)[..., :D], vc.to(device)[..., :D],
-                            table.to(device), lens)
+                            table.to(device), torch.tensor(lens, dtype=torch.int32, device=device))
     keep = torch.ones(lens[0], dtype=torch.bool)
     for pg in (1, 9):
         keep[pg * bs:(pg + 1) * bs] = False
@@ -123,7 +127,27 @@ def test_shares(device, H, KVH, D, q_len, lens, q_dtype):
     """Few tasks over long contexts: the work list split between workgroups and folded."""
     print(f"[case] shares H={H}/{KVH} D={D} q_len={q_len} {q_dtype}", flush=True)
     q, kc, vc, table = make(H, KVH, D, lens, q_len, q_dtype, q_dtype, 16, q_len)
-    check(device, q, kc, vc, table, lens, D)
+    check(device, q, kc, vc, table, lens, D, shares=True)
+
+
+@pytest.mark.parametrize("H,KVH,D,q_len,B,cap,q_dtype,kv_dtype", [
+    (8, 8, 32, 129, 65, 256, F32, F32),     # 1040 tasks, more than a work list holds
+    (8, 8, 32, 129, 65, 256, BF16, BF16),
+    (10, 5, 96, 190, 17, 256, F16, F16),    # 255 tasks, not a multiple of 8: about one a CU
+    (10, 5, 128, 190, 17, 256, F32, BF16),
+    (10, 5, 80, 190, 17, 256, BF16, FP8),
+    (21, 3, 200, 60, 20, 128, BF16, BF16),  # 240 tasks of one key-step pair
+])
+def test_one_task_a_workgroup(device, H, KVH, D, q_len, B, cap, q_dtype, kv_dtype):
+    """The launch without shares: tasks dealt to the XCDs, the grid's tail, contexts of every
+    kind; the last row block holds part of its 128 rows."""
+    print(f"[case] one task H={H}/{KVH} D={D} B={B} {q_dtype}/{kv_dtype}", flush=True)
+    lens = [int(x) for x in torch.randint(1, cap + 1, (B,), generator=torch.Generator().manual_seed(D))]
+    lens[:4] = [cap, 0, q_len - 1, cap - 1]
+    q, kc, vc, table = make(H, KVH, D, lens, q_len, q_dtype, kv_dtype, 16, q_len)
+    table = table[:, :cap // 16].contiguous()
+    check(device, q, kc, vc, table, lens, D, shares=False)
+    check(device, q, kc, vc, table, lens, D, shares=False, window=50)
 
 
 @pytest.mark.parametrize("q_dtype,rows", [(F32, 120), (BF16, 120)])

@@ -87,6 +87,9 @@ CASES = {  # name -> (H, KVH, D, dtype, q_len, first lens, second lens, width in
     "partition fp32": (14, 2, 64, torch.float32, 1, [400, 130, 512, 9], [200, 35], 32),
     "generic fp32": (14, 2, 96, torch.float32, 1, [400, 130, 512, 9], [200, 35], 32),
     "prefill": (28, 4, 128, torch.bfloat16, 64, [512, 700], [64], 48),
+    # the any-layout kernel, whose shares are counted from the workspace's size
+    "any-layout prefill fp32": (28, 4, 128, torch.float32, 128, [900, 1500], [300, 129], 256),
+    "any-layout prefill": (24, 8, 96, torch.bfloat16, 200, [1900], [260, 201], 128),
     # 8 x 4 = 32 rows per KV head over 16 pairs: the partition kernel's 16-row tiles
     "partition prefill": (32, 8, 128, torch.bfloat16, 8, [900, 3000], [100], 256),
 }
@@ -99,6 +102,10 @@ def test_noalloc_matches_workspace_entry(device, name):
         note(f"noalloc {name} call {i + 1}: B={len(lens)} lens={lens}")
         q, kc, vc, table = make(H, KVH, D, lens, q_len, dtype, width, seed=7 * i + len(name))
         max_ctx = width * 16
+        if name.startswith("any-layout"):
+            for size in (None, SCRATCH):
+                assert kernel_route(q.to(device), kc.to(device), table, workspace_bytes=size) == \
+                    "prefill any-layout"
         out_ws, out_na = call_both(device, q, kc, vc, table, lens, max_ctx)
         assert torch.equal(out_ws, out_na)
         check_oracle(out_na, q, kc, vc, table, lens)
