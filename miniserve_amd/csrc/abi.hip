@@ -193,7 +193,12 @@ int mfma_rows_per_tile(int rows_per_kvh) { return rows_per_kvh >= 16 ? 16 : next
 // A multi-token query of more than 16 rows per KV head that the copying prefill kernel cannot
 // take may run on the any-layout prefill kernel (prefill_any.h): its geometry. (Decodes do not:
 // at other head sizes the generic kernel measured 1.3-1.9 times faster on 16-bit caches.)
-constexpr int64_t kPaReserve = 40 << 20;  // bytes of share partials a workspace reserves
+// Bytes of share partials that a workspace of such a chunk holds. Above 128 dims that is fewer
+// shares than CUs (152 at 256 dims, 208 at 192), and a launch of shares leaves CUs idle: 256
+// queries of H32/KVH8/D256 over 1500 keys 74 us, 60 with the 240 shares of 62 MiB (40 shapes of
+// 160 to 256 dims: 40 % less to 8 % more). It stays at what the largest chunks up to 128 dims
+// need, as every workspace and the 64 MiB scratch hold it.
+constexpr int64_t kPaReserve = 40 << 20;
 
 bool prefill_any_ok(int batch, int q_len, int num_heads, int num_kv_heads, int head_dim) {
   return q_len > 1 && head_dim <= kMaxHeadDim && batch <= 65535 &&
@@ -1033,8 +1038,10 @@ bool prefill_any_vec(const void* query, const void* out, int head_dim, bool rows
 // an 8-row, 16-key tile at 96 dims (182 us for 256 queries of H24/KVH8 over 1.8k keys); the
 // any-layout kernel takes those in 580 and 30 us, and where they hold few tiles (one sequence
 // of 49 queries, H14/KVH2/D128, 2000 keys: 30 against 88 us) it idles most CUs and loses.
-// Element loads double a step. Within 15 % the two measured level. Up to 96 rows per KV head, where its 128-row blocks are mostly
-// padding and the fit is coarse, it has to win twofold.
+// Element loads double a step. Within 15 % the two measured level. Up to 96 rows per KV head,
+// where its 128-row blocks are mostly padding and the fit is coarse, it has to win twofold. A
+// window is not counted on either side: the other kernels launch its empty partitions (64 queries
+// of H24/KVH8/D96 under 128 tokens of a 65,536-token table 154 us, 19 here).
 bool prefill_any_preferred(int batch, int q_len, int num_heads, int num_kv_heads, int head_dim,
                            int max_context, int q_dtype, int kv_dtype, bool mfma_decode, bool vec) {
   const int64_t rows = static_cast<int64_t>(q_len) * (num_heads / num_kv_heads);

@@ -820,7 +820,7 @@ hipError_t launch_prefill_any_one(const PrefillParams& p, hipStream_t stream) {
                : launch_prefill_any_vec<T, KT, DP, false>(p, stream);
 }
 
-// Defined per query type in prefill_any_<type>.hip, for every cache type.
+// Defined in prefill_any_<query type>_<cache type>.hip, a file a pair.
 template <typename T, typename KT>
 hipError_t launch_prefill_any(const PrefillParams& p, hipStream_t stream);
 
