@@ -12,9 +12,8 @@
 // fp32: S^T and O^T on v_mfma_f32_32x32x2_f32 (64 cycles for 4096 FLOP, 157 TFLOP/s a chip),
 // which bounds the kernel: at 128 dims a 32-key step holds 8192 such cycles a wave against
 // about 260 of LDS reads and 1000 of softmax. Measured on 2 x 512 queries over 4.6k keys
-// (H28/KVH4/D128, 63.9 GFLOP): 578 us = 110 TFLOP/s, 71 % of the unit's cycles busy (80 % in
-// the key loop: both waves of a SIMD are in their softmax, 1350 cycles of a 20,500-cycle step
-// pair, at about the same time, and 1500 go to the step's loads, buffer writes and barrier).
+// (H28/KVH4/D128, 63.9 GFLOP): 579 us with the fold's 11, 110 TFLOP/s, the matrix unit busy in
+// 71 % of the kernel's cycles, no bank conflicts.
 // The decode partition kernel, which took these calls before at 16 rows a tile and re-reads
 // K and V for every tile, measured 913 us. Tried and not kept: two 4-wave workgroups a CU
 // instead of two key groups (584 us, twice the partials); group 1 half a step behind group 0
@@ -24,13 +23,13 @@
 // 16-bit types: v_mfma_f32_32x32x16. The weights are kept in two operands of the query type,
 // P = hi + lo, so that P V is summed over products as exact as the result's rounding needs (the
 // generic kernel's weights are fp32): 15 to 16 significant bits in bf16, 2^-7 of the result's
-// own rounding; 21 or more in fp16, whose lo is scaled by 2^18 and summed on its own, so that a weight is
-// held to 2^-43 of the row's largest rather than to fp16's smallest step, 2^-24 (a row whose
-// largest weight meets a zero value is made of the small ones). hi is rounded down and lo gets
-// 2^-24 of the weight on top, so that neither is below 0 nor is lo 0 beside a weight: an infinite
-// value then gives an infinite result, not the NaN of inf - inf or inf * 0. 256 queries over 512 to 2304
-// keys (H24/KVH8/D96 bf16): 30 us against the generic kernel's 182; 4 x 256 queries over 4096
-// keys (H32/KVH8/D256): 0.38 ms against 7.5.
+// own rounding; 21 or more in fp16, whose lo is scaled by 2^18 and summed on its own, so that a
+// weight is held to 2^-42 of the row's largest rather than to fp16's smallest step, 2^-24 (a row
+// whose largest weight meets a zero value is made of the small ones). hi is rounded down and lo
+// gets 2^-24 of the weight on top, so that neither is below 0 nor is lo 0 beside a weight: an
+// infinite value then gives an infinite result, not the NaN of inf - inf or inf * 0. 256 queries
+// over 512 to 2304 keys (H24/KVH8/D96 bf16): 30 us against the generic kernel's 182; 4 x 256
+// queries over 4096 keys (H32/KVH8/D256): 0.31 ms in bf16, 0.32 in fp16, against 7.5.
 //
 // Lane layout (both): lane (cc = l % 32, hh = l / 32) holds query row cc. Register v of a
 // 32-key score tile is key (v & 3) + 8 (v >> 2) + 4 hh; register v of output tile t is dim
