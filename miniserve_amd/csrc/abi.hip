@@ -584,9 +584,9 @@ PartialsPlan plan_partials(const void* query, int q_dtype, int kv_dtype, int hea
   // runs start faster.
   const int64_t triples = static_cast<int64_t>(batch) * num_kv_heads * ceil_div(rows, pl.RT);
   const bool merges = has_out && key_lo == 0 && kFusedMerge && triples <= kMaxTickets;
-  // A sliding window counts for what it shows: 32 sequences of 16k tokens under a 1024-token
-  // window (H32/KVH8/D128 fp16) take 30.9 us on stream-K and the merge, 27.7 on the partition
-  // kernel; 64 under a 128-token one 22.1 and 17.6.
+  // A sliding window counts for what it shows: 32 sequences of 2-16k tokens under a 1024-token
+  // window (H32/KVH8/D128 fp16) take 33.5 us on stream-K and the merge, 27.8 on the partition
+  // kernel; 64 under a 128-token one 19.5 and 9.2.
   window = effective_window(window, max_context);
   const bool windowed =
       merges && windows_shrink(kv_dtype == MSATTN_FP8_E4M3, pl.RT, head_dim, window);
@@ -752,10 +752,10 @@ int partials_impl(const void* query, const void* k_cache, const void* v_cache,
     // tiles (wave w owns tiles 8 w .. 8 w + 7), which costs the less the fewer they are of all.
     // Timed both ways on H32/KVH8 and H28/KVH4 at 128 dims and H14/KVH2 at 64, bf16 and fp8
     // caches, contexts of 5/8 of the table up and full ones:
-    //   np >= 3: level to 36 % faster (16 x H28/KVH4 at 3584 tokens 29.2 -> 25.3 us);
+    //   np >= 3: level to 36 % faster (16 x H28/KVH4 at 3584 tokens 32.5 -> 28.7 us);
     //   np == 2: from 7/8 of both partitions, -20 to +4 %; at 1040 tokens up to 34 % slower;
     //   np == 1 (one workgroup a triple, no merge): from half the partition where the launch
-    //     fills 80 to 100 % of the CUs, 2-32 % faster (32 x H32/KVH8 at 512 tokens 17.4 ->
+    //     fills 80 to 100 % of the CUs, 2-32 % faster (32 x H32/KVH8 at 512 tokens 17.3 ->
     //     15.0); with fewer or more triples, or a shorter table, up to 60 % slower in places
     //     (288 x H28/KVH4 pairs at 320 tokens 13.7 -> 21.9 over fp8, 48 x H32/KVH8 at 128
     //     tokens 14.2 -> 16.5).
@@ -788,7 +788,7 @@ int partials_impl(const void* query, const void* k_cache, const void* v_cache,
     // Under a window: the tiles it can touch in equal partitions from its first tile on (never
     // more slots a row than the workspace holds). The empty partitions below the window were
     // launched, stored and merged before: 8 x H28/KVH4/D128, 4 queries over 16k tokens under a
-    // 1024-token window 39.4 -> 21.8 us, one query 23.3 -> 18.3. (The wide shape and the fp32
+    // 1024-token window 36.9 -> 17.8 us, one query 21.5 -> 10.6. (The wide shape and the fp32
     // route's long partitions are still taken by the table, above, and then cut to the window.)
     //
     // Their size, for the regular shape: the smallest whose launch stays within kTargetSlots
