@@ -802,7 +802,9 @@ int partials_impl(const void* query, const void* k_cache, const void* v_cache,
     // smallest size, or at 16 rows a tile: the merge reads them all (4 x H28/KVH4 fp32 under 1590
     // tokens 22.9 us in 26 of 64 tokens, 18.7 in 13 of 128).
     const int64_t shown = static_cast<int64_t>(p.window) + q_len - 1;
-    if (windows_shrink(kv_fp8, RT, head_dim, p.window) && shown < max_context) {
+    // (a window within two tiles of the table's length has nothing worth laying anew; the margin
+    // also keeps the tile counts below 2^31)
+    if (windows_shrink(kv_fp8, RT, head_dim, p.window) && shown + 32 < max_context) {
       const int tiles = ceil_div(static_cast<int>(shown) + 15, 16);
       const int64_t triples = static_cast<int64_t>(batch) * num_kv_heads * p.rtiles;
       int most = p.part;

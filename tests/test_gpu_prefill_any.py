@@ -211,3 +211,42 @@ def test_infinite_values_stay_infinite(device, q_dtype):
         assert bool((out[..., 10] == float("inf")).all()) and bool((out[..., 11] == float("-inf")).all())
         keep = [d for d in range(D) if d not in (10, 11)]
         assert torch.equal(out[..., keep], finite[..., keep])
+
+
+@pytest.mark.parametrize("H,KVH,D,q_len,q_dtype,cap", [
+    (4, 2, 96, 130, BF16, 4096),     # shares and a fold launch
+    (28, 4, 128, 130, F32, 4096),
+    (10, 5, 80, 190, F16, 256),      # one task a workgroup
+])
+def test_captured_chunk_replays_with_new_inputs(device, H, KVH, D, q_len, q_dtype, cap):
+    """A captured chunk over replays with other lengths, tables and queries in its buffers, eager
+    calls on the same workspace between them: each replay the eager call's bits."""
+    B = 17 if cap == 256 else 2
+    print(f"[case] capture H={H}/{KVH} D={D} {q_dtype} cap={cap}", flush=True)
+    g = torch.Generator(device).manual_seed(D)
+    gc = torch.Generator().manual_seed(D)
+    kc, vc = (torch.randn(512, 16, KVH, D, generator=g, device=device).to(q_dtype) for _ in range(2))
+    q = torch.randn(B, q_len, H, D, generator=g, device=device).to(q_dtype)
+    table = torch.randint(0, 512, (B, cap // 16), generator=gc).to(device, torch.int32)
+    lens = torch.randint(1, cap + 1, (B,), generator=gc).to(device, torch.int32)
+    assert kernel_route(q, kc, table) == ROUTE
+    ws = torch.zeros(nat.lib().msattn_workspace_bytes(B, q_len, H, KVH, D, cap), dtype=torch.uint8,
+                     device=device)
+    out = torch.empty_like(q)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        paged_attention(q, kc, vc, table, lens, workspace=ws, out=out)
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        paged_attention(q, kc, vc, table, lens, workspace=ws, out=out)
+    for _ in range(4):
+        q.copy_(torch.randn(q.shape, generator=g, device=device).to(q_dtype))
+        table.copy_(torch.randint(0, 512, table.shape, generator=gc).to(torch.int32))
+        lens.copy_(torch.randint(0, cap + 1, (B,), generator=gc).to(torch.int32))
+        want = paged_attention(q, kc, vc, table, lens, workspace=ws)
+        out.fill_(float("nan"))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)
