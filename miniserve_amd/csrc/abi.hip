@@ -801,12 +801,24 @@ int partials_impl(const void* query, const void* k_cache, const void* v_cache,
     // (25 x 4 fp32 queries of H28/KVH4 under 54 tokens 13.8 against 18.5). At most 16 of the
     // smallest size, or at 16 rows a tile: the merge reads them all (4 x H28/KVH4 fp32 under 1590
     // tokens 22.9 us in 26 of 64 tokens, 18.7 in 13 of 128).
+    // Against the launches laid over the table, 1217 shapes: 0.71 of the time on the mean; four
+    // above 1.06 (to 1.25), all under windows of 2/3 of the table or more whose contexts are
+    // mostly shorter, which the grid cannot know.
     const int64_t shown = static_cast<int64_t>(p.window) + q_len - 1;
     // (a window within two tiles of the table's length has nothing worth laying anew; the margin
     // also keeps the tile counts below 2^31)
     if (windows_shrink(kv_fp8, RT, head_dim, p.window) && shown + 32 < max_context) {
       const int tiles = ceil_div(static_cast<int>(shown) + 15, 16);
       const int64_t triples = static_cast<int64_t>(batch) * num_kv_heads * p.rtiles;
+      // The wide shape only within one round of its one workgroup a CU: 37 x H28/KVH4 over fp8
+      // under 1043 tokens 26.5 us in 296 wide workgroups, 21.6 in 444 regular ones; 74 x
+      // H14/KVH2/D64 under 1274 24.5 and 16.8.
+      if (p.mfma_waves == kWideWaves &&
+          triples * ceil_div(16 * tiles, kPartWide) > static_cast<int64_t>(device_cus())) {
+        p.part = L.part;
+        p.max_parts = L.max_parts;
+        p.mfma_waves = kMfmaWaves;
+      }
       int most = p.part;
       if (p.mfma_waves == kMfmaWaves && p.part == L.part) {
         most = kPartMax;

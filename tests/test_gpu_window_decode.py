@@ -62,6 +62,8 @@ def test_windowed_decode(device, H, KVH, D, B, q_len, pages, q_dtype, kv_dtype, 
     (28, 4, 128, 4, 1, 298, torch.float32, 1590, 128, 4),   # more than 16 of 64
     (32, 8, 128, 2, 4, 350, torch.bfloat16, 2553, 256, 4),  # 16 rows a tile: of 128
     (32, 8, 128, 32, 4, 512, torch.bfloat16, 128, 192, 4),  # every CU has a row: one partition
+    (28, 4, 128, 37, 1, 98, torch.bfloat16, 1043, 384, 4),  # 296 wide ones: a second round
+    (28, 4, 128, 16, 1, 224, torch.bfloat16, 2000, 1024, 8),  # 128 wide ones
     (32, 8, 128, 16, 1, 64, torch.bfloat16, 100, 128, 4),   # half the CUs, two tiles a wave: one
     (32, 8, 128, 2, 1, 64, torch.bfloat16, 100, 64, 4),     # fewer rows: two
 ])
